@@ -350,10 +350,11 @@ class HipBackend:
     # ----------------------------------------------------------- ragged decode
     MAX_HOST_PLANS = 64
 
-    def ragged_target(self, batch: int, kv_heads: int) -> int:
+    def ragged_groups(self, batch: int, kv_heads: int) -> tuple[int, int]:
         """Work-groups per kv head a ragged plan aims for when the caller names
-        none: whole rounds of one work-group per CU, with room to split the long
-        sequences.
+        none: those of one round (a work-group per CU), used where they are even,
+        and several rounds with room to split the long sequences, used where they
+        are not (bt_ragged_plan_rounds).
 
         A batch that (nearly) fills one round keeps one split per sequence, and
         the call lasts as long as one CU takes for its longest sequence: 37 GB/s
@@ -365,24 +366,28 @@ class HipBackend:
         78 / 20 -> 76 / 22 us, 48: 93 / 26 -> 85 / 27, 96: 353 / 72 -> 236 / 53,
         144: 798 / 121 -> 246 / 67, 200: 984 / 143 -> 475 / 103; Hkv = 8, D = 128
         (a round of 32), 32 sequences: 480 / 69 -> 166 / 34 in three rounds,
-        128: 798 / 137 -> 595 / 131 in six."""
+        128: 798 / 137 -> 595 / 131 in six.  Equal lengths are why one round is
+        kept where it is even: 96 sequences of 1,000 tokens take 43 us in one
+        round and 47 us in two."""
         batch = int(batch)
         one = max(1, self.num_cus // max(1, kv_heads))
         if 8 * batch <= 3 * one:
-            return one
+            return one, one
         room = max(one, 64, min(batch // 2, 256))
-        return -(-(batch + room) // one) * one
+        return one, -(-(batch + room) // one) * one
 
     def ragged_plan(self, lens: list[int], kv_heads: int, target_groups: int | None = None):
         """Split plan for a ragged batch from host lengths, as device tables:
         sequence b gets ceil(len_b / T) splits for the smallest token cap T
         whose total fits ``target_groups`` work-groups per kv head (default:
-        ``ragged_target``).  Plans are cached per (lens, target), at
+        ``ragged_groups``).  Plans are cached per (lens, target), at
         most MAX_HOST_PLANS of them (least recently used first out); a plan
         used while a graph is being captured is kept until close()."""
         if target_groups is None:
-            target_groups = self.ragged_target(len(lens), kv_heads)
-        key = (tuple(int(x) for x in lens), int(target_groups))
+            one, target = self.ragged_groups(len(lens), kv_heads)
+        else:
+            one = target = int(target_groups)
+        key = (tuple(int(x) for x in lens), one, target)
         plan = self._pinned_plans.get(key)
         if plan is None:
             plan = self._plans.get(key)
@@ -399,7 +404,7 @@ class HipBackend:
         return plan
 
     def _host_plan(self, key):
-        lens, target_groups = key
+        lens, one, target = key
         batch = len(lens)
         cap = sum(max(1, -(-int(x) // 32)) for x in lens)
         lens_c = (ctypes.c_int32 * batch)(*lens)
@@ -407,29 +412,34 @@ class HipBackend:
         base = (ctypes.c_int32 * batch)()
         count = (ctypes.c_int32 * batch)()
         total = ctypes.c_int32()
-        n = self._lib.bt_ragged_plan(
-            ctypes.addressof(lens_c), batch, int(target_groups), ctypes.addressof(work), cap,
+        n = self._lib.bt_ragged_plan_rounds(
+            ctypes.addressof(lens_c), batch, one, target, ctypes.addressof(work), cap,
             ctypes.addressof(base), ctypes.addressof(count), ctypes.addressof(total),
         )
         if n < 0:
-            check("bt_ragged_plan", n)
+            check("bt_ragged_plan_rounds", n)
         dev = self._dev
         work_t = torch.tensor(list(work)[: 4 * n], dtype=torch.int32).to(dev)
         base_t = torch.tensor(list(base), dtype=torch.int32).to(dev)
         count_t = torch.tensor(list(count), dtype=torch.int32).to(dev)
         return (work_t, n, base_t, count_t, int(total.value))
 
-    def ragged_plan_device(self, seq_len: torch.Tensor, target_groups: int | None = None):
+    def ragged_plan_device(self, seq_len: torch.Tensor, target_groups: int | None = None,
+                           round_groups: int | None = None):
         """The same plan built on the device from the device lengths ``seq_len``
         (B,) int32, on the current stream with no host synchronisation
         (capturable).  Tables are allocated once per (B, target) and kept until
         close(); returns (work, num_work, split_base, split_count, total_splits)
-        with num_work = total_splits = the table capacity max(B, target)."""
+        with num_work = total_splits = the table capacity max(B, target).
+        ``round_groups`` (at most the target, its default): the plan is for that
+        many work-groups where these are even (bt_ragged_plan_rounds)."""
         batch = int(seq_len.numel())
         if target_groups is None:
             raise ValueError("target_groups is required (CUs / kv heads for one round)")
-        cap = max(batch, int(target_groups))
-        key = (batch, int(target_groups))
+        target_groups = int(target_groups)
+        one = target_groups if round_groups is None else min(int(round_groups), target_groups)
+        cap = max(batch, target_groups)
+        key = (batch, target_groups)
         bufs = self._dev_plans.get(key)
         if bufs is None:
             bufs = (torch.empty((cap, 4), dtype=torch.int32, device=self._dev),
@@ -440,11 +450,11 @@ class HipBackend:
         work, base, count, total = bufs
         if seq_len.dtype != torch.int32 or seq_len.device != self._dev or not seq_len.is_contiguous():
             raise RuntimeError("seq_len must be a contiguous int32 device tensor")
-        rc = self._lib.bt_ragged_plan_device(
-            seq_len.data_ptr(), batch, int(target_groups), work.data_ptr(), cap, base.data_ptr(),
+        rc = self._lib.bt_ragged_plan_rounds_device(
+            seq_len.data_ptr(), batch, one, target_groups, work.data_ptr(), cap, base.data_ptr(),
             count.data_ptr(), total.data_ptr(), _stream(self._dev),
         )
-        check("bt_ragged_plan_device", rc)
+        check("bt_ragged_plan_rounds_device", rc)
         return work, cap, base, count, cap
 
     def attention_ragged(
@@ -463,10 +473,11 @@ class HipBackend:
         if seq_offset.dtype != torch.int64 or seq_len.dtype != torch.int32:
             raise RuntimeError("seq_offset must be int64 and seq_len int32")
         q = q.contiguous()
-        if target_groups is None:
-            target_groups = self.ragged_target(batch, groups)
         if lens is None:
-            work, n, base, count, total = self.ragged_plan_device(seq_len, target_groups)
+            one = None
+            if target_groups is None:
+                one, target_groups = self.ragged_groups(batch, groups)
+            work, n, base, count, total = self.ragged_plan_device(seq_len, target_groups, one)
         else:
             work, n, base, count, total = self.ragged_plan(lens, groups, target_groups)
         ws = self._workspace(heads, dim, total)

@@ -231,15 +231,24 @@ inline int decode_mode(bool work, bool pos, bool seq_len, bool seq_offset, int b
   return (batch == 1 && !seq_offset) ? 0 : -1;
 }
 
-// Device-side ragged plan (ragged_plan.hip): the plan bt_ragged_plan makes on
-// the host, from device lengths, padded to work_capacity entries with {-1, ..}.
+// Whether one round of `round` work-groups serves a ragged batch evenly: its n
+// splits, of at most `longest` tokens each, take ceil(n / round) rounds; even
+// means that these hold at most 1.5 times the batch's tokens.
+inline __host__ __device__ bool ragged_round_is_even(int64_t n, int64_t longest, int64_t tokens, int64_t round) {
+  return 2 * ((n + round - 1) / round) * longest * round <= 3 * tokens;
+}
+
+// Device-side ragged plan (ragged_plan.hip): the plan bt_ragged_plan_rounds
+// makes on the host, from device lengths, padded to work_capacity entries with
+// {-1, ..}.
 constexpr int kRaggedPlanMaxBatch = 4096;
 struct RaggedPlanParams {
   const int32_t* seq_len;  // (batch,) device lengths
   int32_t batch;
-  int32_t target_groups;
+  int32_t round_groups;    // work-groups of one round
+  int32_t target_groups;   // work-groups where one round is uneven
   int32_t* work;           // (work_capacity, 4) entries {b, s, ns_b, base_b}
-  int32_t work_capacity;   // >= max(batch, target_groups)
+  int32_t work_capacity;   // >= max(batch, target_groups, round_groups)
   int32_t* split_base;     // (batch,)
   int32_t* split_count;    // (batch,)
   int32_t* total;          // optional: the number of real entries

@@ -326,18 +326,27 @@ int bt_gqa_decode_noalloc(const void* q, int32_t q_dtype, int64_t q_stride_seq, 
 int32_t bt_ragged_plan(const int32_t* lens, int32_t batch, int32_t target_groups, int32_t* work,
                        int32_t work_capacity, int32_t* split_base, int32_t* split_count,
                        int32_t* total_splits) {
+  return bt_ragged_plan_rounds(lens, batch, target_groups, target_groups, work, work_capacity, split_base,
+                               split_count, total_splits);
+}
+
+int32_t bt_ragged_plan_rounds(const int32_t* lens, int32_t batch, int32_t round_groups, int32_t target_groups,
+                              int32_t* work, int32_t work_capacity, int32_t* split_base, int32_t* split_count,
+                              int32_t* total_splits) {
   if (!lens || !work || !split_base || !split_count || !total_splits) return BT_EINVAL;
-  if (batch < 1 || target_groups < 1) return BT_EINVAL;
+  if (batch < 1 || round_groups < 1 || target_groups < 1) return BT_EINVAL;
   int32_t max_len = 1;
+  int64_t tokens = 0;
   for (int32_t b = 0; b < batch; ++b) {
     if (lens[b] < 0) return BT_EINVAL;
     max_len = std::max(max_len, lens[b]);
+    tokens += lens[b];
   }
   // Splits of sequence b under a cap of T tokens per split: ceil(len / T),
   // at least 1, at most one per 32 tokens and kMaxSplitsPerSeq.
   auto splits_of = [](int32_t len, int32_t cap) {
     int64_t ns = ((int64_t)len + cap - 1) / cap;
-    ns = std::min<int64_t>(ns, (len + 31) / 32);
+    ns = std::min<int64_t>(ns, ((int64_t)len + 31) / 32);
     ns = std::min<int64_t>(ns, bt::kMaxSplitsPerSeq);
     return (int32_t)std::max<int64_t>(ns, 1);
   };
@@ -346,17 +355,28 @@ int32_t bt_ragged_plan(const int32_t* lens, int32_t batch, int32_t target_groups
     for (int32_t b = 0; b < batch; ++b) n += splits_of(lens[b], cap);
     return n;
   };
-  // The smallest cap whose split total fits target_groups (the count only
-  // falls as the cap grows): every work-group then streams at most that many
-  // tokens and the batch runs in one round of target_groups work-groups per kv
-  // head.  A batch with more sequences than target_groups gets one split each.
-  int32_t lo = 1, hi = max_len;
-  while (lo < hi) {
-    const int32_t mid = lo + (hi - lo) / 2;
-    if (count_at(mid) <= target_groups) hi = mid;
-    else lo = mid + 1;
+  // The smallest cap whose split total fits `target` (the count only falls as
+  // the cap grows): every work-group then streams at most that many tokens and
+  // the batch runs in rounds of work-groups per kv head.  A batch with more
+  // sequences than `target` gets one split each.
+  auto cap_for = [&](int32_t target) {
+    int32_t lo = 1, hi = max_len;
+    while (lo < hi) {
+      const int32_t mid = lo + (hi - lo) / 2;
+      if (count_at(mid) <= target) hi = mid;
+      else lo = mid + 1;
+    }
+    return lo;
+  };
+  int32_t cap = cap_for(round_groups);
+  if (target_groups != round_groups) {
+    int64_t longest = 0;
+    for (int32_t b = 0; b < batch; ++b) {
+      const int64_t ns = splits_of(lens[b], cap);
+      longest = std::max(longest, (lens[b] + ns - 1) / ns);
+    }
+    if (!bt::ragged_round_is_even(count_at(cap), longest, tokens, round_groups)) cap = cap_for(target_groups);
   }
-  const int32_t cap = lo;
   int32_t total = 0;
   for (int32_t b = 0; b < batch; ++b) {
     const int32_t ns = splits_of(lens[b], cap);
@@ -389,13 +409,21 @@ int32_t bt_ragged_plan(const int32_t* lens, int32_t batch, int32_t target_groups
 int bt_ragged_plan_device(const int32_t* seq_len, int32_t batch, int32_t target_groups, int32_t* work,
                           int32_t work_capacity, int32_t* split_base, int32_t* split_count,
                           int32_t* total_splits, void* stream) {
+  return bt_ragged_plan_rounds_device(seq_len, batch, target_groups, target_groups, work, work_capacity, split_base,
+                                      split_count, total_splits, stream);
+}
+
+int bt_ragged_plan_rounds_device(const int32_t* seq_len, int32_t batch, int32_t round_groups, int32_t target_groups,
+                                 int32_t* work, int32_t work_capacity, int32_t* split_base, int32_t* split_count,
+                                 int32_t* total_splits, void* stream) {
   if (!seq_len || !work || !split_base || !split_count) return BT_EINVAL;
-  if (batch < 1 || target_groups < 1 || !aligned16(work)) return BT_EINVAL;
+  if (batch < 1 || round_groups < 1 || target_groups < 1 || !aligned16(work)) return BT_EINVAL;
   if (batch > bt::kRaggedPlanMaxBatch) return BT_ENOTSUP;
-  if (work_capacity < std::max(batch, target_groups)) return BT_ENOSPC;
+  if (work_capacity < std::max(batch, std::max(round_groups, target_groups))) return BT_ENOSPC;
   bt::RaggedPlanParams p{};
   p.seq_len = seq_len;
   p.batch = batch;
+  p.round_groups = round_groups;
   p.target_groups = target_groups;
   p.work = work;
   p.work_capacity = work_capacity;

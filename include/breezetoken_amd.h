@@ -131,6 +131,15 @@ int32_t bt_ragged_plan(const int32_t* lens, int32_t batch, int32_t target_groups
                        int32_t* work, int32_t work_capacity, int32_t* split_base,
                        int32_t* split_count, int32_t* total_splits);
 
+/* The same with two sizes: the plan for `round_groups` work-groups per kv head
+ * where it is even -- the rounds of round_groups that its splits take, of the
+ * longest split's tokens each, hold at most 1.5 times the batch's tokens --
+ * and the plan for `target_groups` where it is not.  bt_ragged_plan is
+ * round_groups = target_groups. */
+int32_t bt_ragged_plan_rounds(const int32_t* lens, int32_t batch, int32_t round_groups,
+                              int32_t target_groups, int32_t* work, int32_t work_capacity,
+                              int32_t* split_base, int32_t* split_count, int32_t* total_splits);
+
 /* Device-side planner for ragged batches: the plan bt_ragged_plan makes, built
  * on `stream` from the device lengths seq_len[batch] (negative lengths count
  * as 0), so a decode step over many growing sequences needs no host
@@ -145,6 +154,13 @@ int32_t bt_ragged_plan(const int32_t* lens, int32_t batch, int32_t target_groups
 int bt_ragged_plan_device(const int32_t* seq_len, int32_t batch, int32_t target_groups,
                           int32_t* work, int32_t work_capacity, int32_t* split_base,
                           int32_t* split_count, int32_t* total_splits, void* stream);
+
+/* The plan bt_ragged_plan_rounds makes, built on the device (work_capacity >=
+ * max(batch, round_groups, target_groups)). */
+int bt_ragged_plan_rounds_device(const int32_t* seq_len, int32_t batch, int32_t round_groups,
+                                 int32_t target_groups, int32_t* work, int32_t work_capacity,
+                                 int32_t* split_base, int32_t* split_count, int32_t* total_splits,
+                                 void* stream);
 
 /* Ragged multi-sequence decode over one shared cache: sequence b occupies
  * slots [seq_offset[b], seq_offset[b] + seq_len[b]).  `work`, split_base and
