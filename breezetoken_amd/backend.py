@@ -333,7 +333,7 @@ class HipBackend:
         batch, heads, dim = q.shape
         groups = self._check_kv(k, v, heads, dim)
         q = q.contiguous()
-        ns = max(1, self.pick_splits(groups * batch, max_len))
+        ns = int(self._lib.bt_decode_pick_splits_batch(batch, heads, groups, min(int(max_len), 0x7FFFFFFF), self.num_cus))
         ws = self._workspace(heads, dim, batch * ns)
         out = torch.empty((batch, heads, dim), dtype=torch.float32, device=self._dev)
         rc = self._lib.bt_gqa_decode(

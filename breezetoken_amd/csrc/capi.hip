@@ -168,6 +168,36 @@ int32_t bt_decode_pick_splits(int32_t kv_heads, int32_t ctx_len, int32_t num_cus
   return ns < 1 ? 1 : ns;
 }
 
+int32_t bt_decode_pick_splits_batch(int32_t batch, int32_t heads, int32_t kv_heads, int32_t max_len,
+                                    int32_t num_cus) {
+  if (batch < 1) batch = 1;
+  if (kv_heads < 1) kv_heads = 1;
+  if (heads < kv_heads) heads = kv_heads;
+  if (num_cus < 1) num_cus = 256;
+  if (max_len < 1) max_len = 1;
+  const int64_t pairs = (int64_t)batch * kv_heads, cus = num_cus;
+  // The time of ns splits in tokens of one CU's stream: a work-group streams
+  // max_len / ns tokens and costs as much as kFixed + 2 * group more (prologue,
+  // merge; its partials' way through memory); work-groups run in rounds of one
+  // per CU, and a round that is not full is hardly faster (a CU alone reads 26
+  // GB/s against 23 GB/s with all of them streaming); a quarter of a
+  // work-group stands for the lengths' spread at the end.
+  constexpr int64_t kFixed = 80;
+  const int64_t fixed = kFixed + 2 * (heads / kv_heads);
+  const int64_t tiles = (max_len + 31) / 32;
+  const int64_t most = std::min<int64_t>(std::min<int64_t>(tiles, bt::kMaxSplitsPerSeq), 1 + 4 * cus / pairs);
+  int64_t best = 1, best_cost = INT64_MAX;
+  for (int64_t ns = 1; ns <= most; ++ns) {
+    const int64_t groups = pairs * ns, share = max_len / ns, full = groups / cus;
+    const int64_t cost = full * (fixed + share) + (groups % cus ? fixed + share * 9 / 10 : 0) + share / 4;
+    if (cost < best_cost) {
+      best = ns;
+      best_cost = cost;
+    }
+  }
+  return (int32_t)best;
+}
+
 int bt_gqa_decode_split(const void* q, int32_t q_dtype, int64_t q_stride_seq, const void* k,
                         const void* v, int64_t kv_stride_tok, int64_t kv_stride_head,
                         const int64_t* seq_offset, const int32_t* pos, const int32_t* seq_len,

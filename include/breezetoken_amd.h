@@ -55,6 +55,17 @@ int64_t bt_decode_workspace_bytes(int32_t heads, int32_t head_dim, int32_t total
  * `num_cus` compute units (the reference hard-codes 16, backends.py:526,550). */
 int32_t bt_decode_pick_splits(int32_t kv_heads, int32_t ctx_len, int32_t num_cus);
 
+/* Uniform split count for `batch` sequences of up to max_len tokens that share
+ * one call (bt_gqa_decode's batch modes): the count whose rounds of work-groups
+ * (batch * kv_heads * splits, one per CU at a time) finish first by a model of
+ * a work-group's stream and fixed cost.  bt_decode_pick_splits rounds up to a
+ * work-group per CU instead, which leaves a second, nearly empty round where
+ * batch * kv_heads does not divide the CUs: 24 sequences of 3,000 tokens, Hkv =
+ * 2, D = 256: 43.2 us with 6 splits (288 work-groups), 31.3 us with 5 (240);
+ * Hkv = 8, D = 128: 67.9 us with 2 (384), 57.3 us with 4 (768). */
+int32_t bt_decode_pick_splits_batch(int32_t batch, int32_t heads, int32_t kv_heads,
+                                    int32_t max_len, int32_t num_cus);
+
 /* Tokens per tile.  The split pass deals tiles to splits round-robin: tile t
  * (tokens [t*T, (t+1)*T)) belongs to split t % num_split.  The reference gives
  * each split a contiguous range instead (attention.py:106-112); the combined
