@@ -292,7 +292,17 @@ class HipBackend:
         if q.device != self._dev:
             raise RuntimeError("q must live on the backend's device")
         q = q.contiguous()
-        ns = self._lib.bt_decode_pick_splits(groups, slots, self.num_cus)
+        # One split writes the result itself and needs no combine.  It is as
+        # fast up to a tile or two per wave -- D = 256 / 128 / 64: 128 / 256 /
+        # 448 keys, 5.7 / 5.1 / 4.6 us a graph node against 5.7 / 5.3 / 4.9 --
+        # and where the calls are issued one by one, whose 2.6 us per launch
+        # outlast the kernels, up to 320 / 640 / 1280 keys: 301 / 512 / 1024
+        # keys 10.2 / 11.4 / 10.1 -> 8.7 / 8.0 / 7.4 us.
+        size = slots * dim
+        if size <= 32768 or (size <= 81920 and pos is None and not torch.cuda.is_current_stream_capturing()):
+            ns = 1
+        else:
+            ns = self._lib.bt_decode_pick_splits(groups, slots, self.num_cus)
         ws = self._workspace(heads, dim, ns)
         out = torch.empty((heads, dim), dtype=torch.float32, device=self._dev)
         row = heads * dim

@@ -34,6 +34,11 @@ struct DecodeSplitParams {
   float* lse;                // (heads, total_splits)
   float* part;               // (heads, total_splits, D)
   int32_t tiles_per_split;   // > 0: a sequence of n tiles uses min(num_split, ceil(n / this)) splits
+  // Set where every sequence has one split: the split's rows are the results
+  // and go here, (batch, heads, D) f32 or bf16, instead of to part and lse.
+  void* out;
+  int out_bf16;
+  int64_t out_stride_seq;
 };
 
 // Waves per decode split work-group, and the tiles per split below which

@@ -181,15 +181,17 @@ int32_t bt_decode_pick_splits_batch(int32_t batch, int32_t heads, int32_t kv_hea
   // merge; its partials' way through memory); work-groups run in rounds of one
   // per CU, and a round that is not full is hardly faster (a CU alone reads 26
   // GB/s against 23 GB/s with all of them streaming); a quarter of a
-  // work-group stands for the lengths' spread at the end.
-  constexpr int64_t kFixed = 80;
+  // work-group stands for the lengths' spread at the end; more than one split
+  // costs the combine's launch.
+  constexpr int64_t kFixed = 80, kCombine = 64;
   const int64_t fixed = kFixed + 2 * (heads / kv_heads);
   const int64_t tiles = (max_len + 31) / 32;
   const int64_t most = std::min<int64_t>(std::min<int64_t>(tiles, bt::kMaxSplitsPerSeq), 1 + 4 * cus / pairs);
   int64_t best = 1, best_cost = INT64_MAX;
   for (int64_t ns = 1; ns <= most; ++ns) {
     const int64_t groups = pairs * ns, share = max_len / ns, full = groups / cus;
-    const int64_t cost = full * (fixed + share) + (groups % cus ? fixed + share * 9 / 10 : 0) + share / 4;
+    const int64_t cost = full * (fixed + share) + (groups % cus ? fixed + share * 9 / 10 : 0) + share / 4 +
+                         (ns > 1 ? kCombine : 0);
     if (cost < best_cost) {
       best = ns;
       best_cost = cost;
@@ -286,8 +288,15 @@ int bt_gqa_decode(const void* q, int32_t q_dtype, int64_t q_stride_seq, const vo
   // A short context in a large grid uses fewer, fuller splits (the split count
   // follows the length on the device; the combine skips the empty splits).
   p.tiles_per_split = bt::kDecodeTilesPerSplit;
+  if (num_split == 1) {
+    // The only split's rows are the results (the combine would weigh them by
+    // 2^0 / 1), so it writes them and no combine is launched.
+    p.out = out;
+    p.out_bf16 = out_dtype == BT_DTYPE_BF16;
+    p.out_stride_seq = out_stride_seq > 0 ? out_stride_seq : (int64_t)heads * head_dim;
+  }
   rc = hip_rc(bt::launch_decode_split(p, head_dim, num_split, batch, (hipStream_t)stream));
-  if (rc) return rc;
+  if (rc || num_split == 1) return rc;
   return bt_gqa_decode_combine(lse, part, batch, heads, head_dim, num_split, nullptr, nullptr,
                                total, out, out_dtype, out_stride_seq, stream);
 }

@@ -115,7 +115,11 @@ enum DecodeMode : int {
 // LDS, and its next K as soon as Q.K^T has consumed the current one -- except
 // after the first tile, where the next K goes out with the next V.  A wave's
 // first tile is requested after its slice of Q^T is built (wave 0's, at entry).
-template <int GMAX, int D, int W, int MODE, bool QBF16>
+//
+// ONE: every sequence has one split, whose merged rows are the results: they go
+// to p.out and no combine follows.  Its own instantiation, so the split kernel
+// keeps its arguments and registers.
+template <int GMAX, int D, int W, int MODE, bool QBF16, bool ONE>
 __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplitParams p) {
   constexpr int kThreads = W * 64;
   constexpr int kSteps = D / 32;            // K-dimension steps of Q.K^T
@@ -284,7 +288,21 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
       ns_eff = want < 1 ? 1 : (want < ns ? want : ns);
     }
   }
+  auto store_out = [&](int h, int d, const float4& a) {
+    const int64_t row = (int64_t)b * p.out_stride_seq + (int64_t)(head0 + h) * D + d;
+    if (p.out_bf16) {
+      const u32x2 pk = {f32x2_to_bf16x2_bits(a.x, a.y), f32x2_to_bf16x2_bits(a.z, a.w)};
+      *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.out) + row) = pk;
+    } else {
+      *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.out) + row) = a;
+    }
+  };
   if (s >= ns_eff || s >= tiles) {
+    if constexpr (ONE) {  // no keys: zeros, as the combine gives
+      for (int item = threadIdx.x; item < G * (D / 4); item += kThreads)
+        store_out(item / (D / 4), (item % (D / 4)) * 4, float4{0.f, 0.f, 0.f, 0.f});
+      return;
+    }
     if (threadIdx.x < G) p.lse[(int64_t)(head0 + threadIdx.x) * p.total_splits + split_idx] = -INFINITY;
     return;
   }
@@ -493,6 +511,10 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
       const bool has = lsum > 0.f;
       const float inv = has ? 1.f / lsum : 0.f;
       acc.x *= inv; acc.y *= inv; acc.z *= inv; acc.w *= inv;
+      if constexpr (ONE) {
+        store_out(h, d, acc);
+        continue;
+      }
       *reinterpret_cast<float4*>(p.part + row * D + d) = acc;
       if (d == 0) p.lse[row] = has ? fast_log2(lsum) + mx : -INFINITY;
     }
@@ -623,9 +645,15 @@ __global__ __launch_bounds__(64) void gqa_decode_combine_kernel(CombineParams p)
 
 template <int GMAX, int D, int MODE, bool QBF16>
 static hipError_t launch_split_t(const DecodeSplitParams& p, int grid_x, int batch, hipStream_t stream) {
-  const dim3 grid(grid_x * p.kv_heads, 1, batch);
-  hipLaunchKernelGGL((gqa_decode_split_kernel<GMAX, D, kDecodeWaves, MODE, QBF16>), grid, dim3(kDecodeWaves * 64), 0,
-                     stream, p);
+  const dim3 grid(grid_x * p.kv_heads, 1, batch), block(kDecodeWaves * 64);
+  if constexpr (MODE != kModeRagged) {
+    if (p.out) {
+      if (p.num_split != 1 || grid_x != 1) return hipErrorInvalidValue;
+      hipLaunchKernelGGL((gqa_decode_split_kernel<GMAX, D, kDecodeWaves, MODE, QBF16, true>), grid, block, 0, stream, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((gqa_decode_split_kernel<GMAX, D, kDecodeWaves, MODE, QBF16, false>), grid, block, 0, stream, p);
   return hipGetLastError();
 }
 

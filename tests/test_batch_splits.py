@@ -15,7 +15,8 @@ from breezetoken_amd import _lib
     (24, 32, 8, 3000, 4),    # 768 in three rounds
     (64, 8, 2, 400, 2),      # short: one round
     (1, 8, 2, 1, 1),
-    (1, 8, 2, 65, 3),        # at most a split per 32 tokens
+    (1, 8, 2, 65, 1),        # one split needs no combine
+    (1, 8, 2, 1000, 32),     # at most a split per 32 tokens
     (5000, 8, 2, 8192, 1),
     (0, 0, 0, 0, 1),         # out-of-range sizes are clamped, as bt_decode_pick_splits does
 ])

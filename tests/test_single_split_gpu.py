@@ -1,0 +1,61 @@
+"""Decode calls with one split, whose kernel writes the result itself: bit for bit
+what the split kernel and the combine give for one split, and the oracle."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from breezetoken_amd import _lib
+from breezetoken_amd import workloads as wl
+from oracle import attention as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,kv,dim", [(8, 2, 256), (16, 2, 128), (6, 2, 64)])
+@pytest.mark.parametrize("seq", [1, 16, 17, 128, 129, 320])
+@pytest.mark.parametrize("q_dtype", [torch.float32, torch.bfloat16])
+def test_eager_single_split_equals_split_and_combine(hip_backend, heads, kv, dim, seq, q_dtype):
+    case = wl.decode_inputs(31, heads, kv, dim, seq, seq)
+    q, k, v = case.q.to(q_dtype).cuda(), case.k.cuda(), case.v.cuda()
+    out = hip_backend.attention(q, k, v, case.scale)
+    assert torch.equal(out, hip_backend.combine(*hip_backend.decode_partials(q, k, v, case.scale, 1)))
+    ref = orc.torch_attention(case.q.float(), case.k.float(), case.v.float(), case.scale)
+    err, cos = orc.compare(out.cpu().numpy(), ref.numpy())
+    # q and P carry 16 bits, sums are f32: 2^-16 of |v| sums to about 1e-4 at most
+    assert err <= 2e-4 and cos >= 0.999999, (err, cos)
+
+
+@pytest.mark.parametrize("out_dtype", [_lib.BT_DTYPE_F32, _lib.BT_DTYPE_BF16])
+def test_batch_single_split_rows_and_empty_sequences(hip_backend, out_dtype):
+    """Three sequences with rows of their own in a wider output, one of them empty."""
+    lens, H, G, D = [33, 0, 100], 8, 2, 256
+    case = wl.c5_inputs(lens=[max(n, 1) for n in lens])
+    q, k, v = case.q.float().cuda(), case.k.cuda(), case.v.cuda()
+    off = torch.tensor(case.offsets, dtype=torch.int64, device="cuda")
+    n = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    tdt = torch.float32 if out_dtype == _lib.BT_DTYPE_F32 else torch.bfloat16
+    wide = H * D + 64
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    outs = []
+    for seq_len, pos in ((n, None), (None, n - 1)):
+        out = torch.full((3, wide), 7.0, dtype=tdt, device="cuda")
+        nbytes = int(lib.bt_decode_workspace_bytes(H, D, 3))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        _lib.check("bt_gqa_decode", lib.bt_gqa_decode(
+            q.data_ptr(), _lib.BT_DTYPE_F32, H * D, k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), off.data_ptr(),
+            None if pos is None else pos.data_ptr(), None if seq_len is None else seq_len.data_ptr(), k.shape[0],
+            3, H, G, D, 1, case.scale, ws.data_ptr(), nbytes, out.data_ptr(), out_dtype, wide, stream))
+        torch.cuda.synchronize()
+        outs.append(out.float().cpu())
+        assert (outs[-1][:, H * D :] == 7.0).all()
+    assert torch.equal(outs[0], outs[1])
+    rows = outs[0][:, : H * D].view(3, H, D)
+    assert (rows[1] == 0).all()
+    for b in (0, 2):
+        o, m = case.offsets[b], lens[b]
+        ref = orc.torch_attention(case.q[b].float(), case.k[o : o + m].float(), case.v[o : o + m].float(), case.scale)
+        err, _ = orc.compare(rows[b].numpy(), ref.numpy())
+        # as above; a bf16 result adds 2^-9 of values below 4
+        assert err <= (2e-4 if tdt == torch.float32 else 8e-3), err
