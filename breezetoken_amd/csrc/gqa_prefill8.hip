@@ -412,7 +412,11 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
               o[m] = to_f16(__uint_as_float((i & 1) ? (w0 & 0xffff0000u) : (w0 << 16)),
                             __uint_as_float((i & 1) ? (w1 & 0xffff0000u) : (w1 << 16)), e);
             }
-            *reinterpret_cast<u32x4*>(v_buf(bsel) + (c * D + dc * 8 + i) * 16) = o;
+            // Row i of the slice in slot i ^ (dc & 7): a wave's lanes write the
+            // same row of neighbouring slices, 128 bytes apart, and would
+            // otherwise meet in two of the 16 bank groups (config 4, S = 64 /
+            // 333 / 500, bf16 q: 10.7 / 18.3 / 19.0 -> 10.3 / 17.8 / 18.5 us).
+            *reinterpret_cast<u32x4*>(v_buf(bsel) + (c * D + dc * 8 + (i ^ (dc & 7))) * 16) = o;
           }
         } else {
           const int e = dek[b];
@@ -467,13 +471,21 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
     };
     // O^T += V^T . P^T over the 64 keys of V^T buffer b: A operand of key half kh
     // / d tile dt is chunk kh*4 + g4 of row dt*16 + i16.
+    // Row d = dt*16 + i16 lies in slot d, in a DIRECT tile with its low bits
+    // turned by those of d / 8 (see write_tiles); its offset in the 16 rows of
+    // d tile dt then depends on dt mod 4.
+    uint32_t v_row[DIRECT ? 4 : 1];
+  #pragma unroll
+    for (int m = 0; m < (DIRECT ? 4 : 1); ++m)
+      v_row[m] = (uint32_t)(DIRECT ? (i16 & 8) + ((i16 & 7) ^ (i16 >> 3) ^ (2 * m)) : i16);
     auto pv = [&](auto b, const u32x4 (&pp)[2]) {
       const unsigned char* vb_ = v_buf(b);
   #pragma unroll
       for (int kh = 0; kh < 2; ++kh) {
   #pragma unroll
         for (int dt = 0; dt < kDTiles; ++dt) {
-          const u32x4 a = *reinterpret_cast<const u32x4*>(vb_ + ((kh * 4 + g4) * D + dt * 16 + i16) * 16);
+          const u32x4 a = *reinterpret_cast<const u32x4*>(
+              vb_ + ((kh * 4 + g4) * D + dt * 16 + v_row[DIRECT ? dt & 3 : 0]) * 16);
           oacc[dt] = mfma16_f16(a, pp[kh], oacc[dt]);
         }
       }
