@@ -97,8 +97,10 @@ struct PrefillParams {
   int32_t kb_chunk;
   // split_compact = 1: the uniform split's grid x lists only the (chunk, kv
   // head subset, query block) items that have keys, each chunk's query blocks
-  // padded to a multiple of 8 (grid y = z = 1); 0: grid (query blocks, kv
-  // heads x subsets, max_chunks), the items past a query block's keys exiting.
+  // padded to a multiple of 8 (grid y = z = 1); 2: the items of at most two
+  // chunks, longest first over all subsets (longest_ahead in gqa_prefill8.hip); 0: grid (query
+  // blocks, kv heads x subsets, max_chunks), the items past a query block's
+  // keys exiting.
   int32_t split_compact;
   // Paired split (pair_parts > 0, kb_chunk = 0): query blocks nqb-1-r and r
   // form pair r; the pair's key blocks (those of nqb-1-r, then those of r) are
@@ -115,17 +117,19 @@ struct PrefillParams {
 // per query block would leave CUs idle (short prompts, long cached prefixes).
 struct PrefillSplitPlan {
   int32_t kb_chunk = 0;    // 0: no uniform split
-  int32_t compact = 0;     // uniform split on the compact grid (see PrefillParams)
+  int32_t compact = 0;     // uniform split on a compact grid (split_compact of PrefillParams)
   int32_t pair_parts = 0;  // 0: no paired split
   int32_t max_chunks = 1;
   int32_t query_blocks = 0;
   size_t part_rows = 0;    // kv_heads x query_blocks x max_chunks x rows per work-group
   size_t part_bytes = 0;   // part_rows x (head_dim f32 partials + 1 f32 LSE)
+  float busiest = 0;       // estimate: key blocks of the busiest CU, its fixed costs among them
   bool active() const { return kb_chunk > 0 || pair_parts > 0; }
-  bool uses_partials() const { return kb_chunk > 0 || (pair_parts > 0 && max_chunks > 1); }
+  bool uses_partials() const { return active() && max_chunks > 1; }
 };
+// `partials` false: only plans that need none.
 PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv_heads, int head_dim,
-                                     int num_cus);
+                                     int num_cus, bool partials);
 
 // Per-row RMSNorm + RoPE (row mode) and the fused decode-step preparation
 // (attention mode); see attn_prep.hip.
@@ -271,7 +275,8 @@ int prefill8_sub_group(int group);
 // Pair kernel (gqa_prefill_pair.hip): two query blocks per work-group, 32
 // query columns per wave; group sizes 1, 2, 4, 8.
 bool prefill_pair_serves(int group, int head_dim);
-int prefill_pair_grid(int seqlen, int group, int kv_heads);
+// Work-groups of a launch and the steps each takes.
+int prefill_pair_grid(int seqlen, int q_offset, int group, int kv_heads, bool q_f32, int* steps);
 hipError_t launch_prefill_pair(const PrefillParams& p, int head_dim, hipStream_t stream);
 // Scaled fp16 V^T image + per-block exponents (p.vt, p.vexp) in the key order
 // of the 16x16 MFMA result layout, and the scaled fp16 K image + exponents

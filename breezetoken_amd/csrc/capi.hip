@@ -112,26 +112,50 @@ int64_t prefill_base_bytes(int32_t kv_len, int32_t kv_heads, int32_t head_dim) {
   return prefill_layout(kv_len, kv_heads, head_dim).bytes;
 }
 
-// Long prompts whose pair grid fills the device run the pair kernel (it needs
-// no split-key partials).
-bool prefill_uses_pair(int32_t seqlen, int32_t heads, int32_t kv_heads, int32_t head_dim) {
-  const int group = heads / kv_heads;
-  if (!bt::prefill_pair_serves(group, head_dim)) return false;
-  return bt::prefill_pair_grid(seqlen, group, kv_heads) >= device_cus();
-}
-
-// The split-key plan bt_gqa_prefill uses for this shape on the current device
-// (kb_chunk 0: none), and where its partials start in the workspace.
-bt::PrefillSplitPlan prefill_plan(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads,
-                                  int32_t head_dim, int64_t* part_offset) {
-  *part_offset = align256(prefill_base_bytes(q_offset + seqlen, kv_heads, head_dim));
+// The split-key plan of the two-waves-per-SIMD kernel for this shape on the
+// current device (inactive: a work-group per query block), without `partials`
+// one that needs none.
+bt::PrefillSplitPlan prefill8_plan(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads,
+                                   int32_t head_dim, bool partials = true) {
   const int group = heads / kv_heads;
   if (!bt::prefill8_serves(group, head_dim)) return bt::PrefillSplitPlan{};
-  if (prefill_uses_pair(seqlen, heads, kv_heads, head_dim)) return bt::PrefillSplitPlan{};
   // The kernel runs the group as subsets of sub_group heads, each subset a
   // row of the grid like a kv head of its own.
   const int sub = bt::prefill8_sub_group(group);
-  return bt::prefill8_split_plan(seqlen, q_offset, sub, kv_heads * (group / sub), head_dim, device_cus());
+  return bt::prefill8_split_plan(seqlen, q_offset, sub, kv_heads * (group / sub), head_dim, device_cus(),
+                                 partials);
+}
+
+// Whether the pair kernel serves this call faster than the two-waves-per-SIMD
+// kernel under `plan`, both estimated in microseconds.  The pair kernel's
+// work-groups all take the same steps of 32 keys and run one per CU, so its
+// time is a whole number of rounds, and a grid just past one costs two: at S =
+// 4500 it took 257 us against 187 (H = 16, Hkv = 2, D = 256, bf16 q), 182
+// against 117 (D = 128).  Within one round it is the faster one once its steps
+// outweigh its start and final merge: bf16 q, H = 8, S = 6000 / 8192 180 /
+// 255 against 181 / 283 us; f32 q, whose pair work-groups are half as large,
+// H = 8, S = 3001 82 against 100, H = 16, S = 1500 53 against 67 us.  The
+// constants (us per call, per step, per 64-key block) fit these and S = 1024
+// .. 8192 at four shapes to about 10%.
+bool prefill_pair_faster(const bt::PrefillSplitPlan& plan, int32_t seqlen, int32_t q_offset, int32_t heads,
+                         int32_t kv_heads, int32_t head_dim, bool q_f32) {
+  const int group = heads / kv_heads;
+  if (!bt::prefill_pair_serves(group, head_dim)) return false;
+  const bool wide = head_dim == 256;
+  const int64_t cus = device_cus();
+  int steps = 0;
+  const int64_t groups = bt::prefill_pair_grid(seqlen, q_offset, group, kv_heads, q_f32, &steps);
+  double rounds = (double)((groups + cus - 1) / cus);
+  // At D = 128 two f32-q work-groups fit a CU and take 1.4 times one's time;
+  // half-filled rounds of two pass as such.
+  if (!wide && q_f32 && groups > cus) rounds = 1.4 * std::max(1.0, 0.5 * (double)((groups + cus - 1) / cus));
+  const double base = wide ? (q_f32 ? 17.0 : 18.0) : (q_f32 ? 11.0 : 13.0);
+  const double step = wide ? (q_f32 ? 1.42 : 1.7) : (q_f32 ? 0.97 : 1.2);
+  const double block = wide ? (q_f32 ? 2.55 : 2.05) : (q_f32 ? 1.36 : 1.14);
+  // Short prompts whose work-groups convert their own blocks have no pre-pass.
+  const int64_t longest = ((int64_t)q_offset + seqlen + bt::kPrefillKeyBlock - 1) / bt::kPrefillKeyBlock;
+  const double base8 = (plan.kb_chunk > 0 ? plan.kb_chunk : longest) <= 2 ? 4.0 : 10.0;
+  return base + rounds * steps * step < 0.95 * (base8 + plan.busiest * block);
 }
 
 }  // namespace
@@ -515,9 +539,8 @@ int64_t bt_prefill_split_workspace_bytes(int32_t seqlen, int32_t q_offset, int32
   if (seqlen < 1 || q_offset < 0 || heads < 1 || kv_heads < 1 || heads % kv_heads || head_dim < 1) return 0;
   if ((int64_t)q_offset + seqlen > INT32_MAX) return 0;
   const int64_t vt = prefill_base_bytes(q_offset + seqlen, kv_heads, head_dim);
-  int64_t part_offset = 0;
-  const bt::PrefillSplitPlan plan = prefill_plan(seqlen, q_offset, heads, kv_heads, head_dim, &part_offset);
-  return plan.uses_partials() ? part_offset + (int64_t)plan.part_bytes : vt;
+  const int64_t part = bt_prefill_partials_bytes(seqlen, q_offset, heads, kv_heads, head_dim);
+  return part > 0 ? align256(vt) + part : vt;
 }
 
 // Shared by bt_gqa_prefill and bt_gqa_prefill_cached: validates the call and
@@ -582,18 +605,19 @@ static int prefill_run(const void* q, int32_t q_dtype, const void* k, const void
   p.img_first = img_first_key / bt::kPrefillKeyBlock;
   p.q_f32 = q_dtype == BT_DTYPE_F32 ? 1 : 0;
   p.keep_images = keep_images ? 1 : 0;
-  if (prefill_uses_pair(seqlen, heads, kv_heads, head_dim))
+  bt::PrefillSplitPlan plan = prefill8_plan(seqlen, q_offset, heads, kv_heads, head_dim);
+  if (plan.uses_partials() && !(partials && partials_bytes >= (int64_t)plan.part_bytes))
+    plan = prefill8_plan(seqlen, q_offset, heads, kv_heads, head_dim, false);
+  if (prefill_pair_faster(plan, seqlen, q_offset, heads, kv_heads, head_dim, p.q_f32 != 0))
     return hip_rc(bt::launch_prefill_pair(p, head_dim, (hipStream_t)stream));
   // Every other shape runs two waves per SIMD (groups of 3, 5, 6, 7 as
   // subsets of 1 or 2 heads).  When one work-group per query block would
-  // leave CUs idle or the causal triangle's work is uneven, and `partials`
-  // holds the plan's partials (if it needs any), the key ranges are split.
+  // leave CUs idle or the causal triangle's work is uneven, the key ranges are
+  // split.
   if (bt::prefill8_serves(p.group, head_dim)) {
     p.sub_group = bt::prefill8_sub_group(p.group);
     p.head_subs = p.group / p.sub_group;
-    int64_t part_offset = 0;
-    const bt::PrefillSplitPlan plan = prefill_plan(seqlen, q_offset, heads, kv_heads, head_dim, &part_offset);
-    if (plan.active() && (!plan.uses_partials() || (partials && partials_bytes >= (int64_t)plan.part_bytes))) {
+    if (plan.active()) {
       p.kb_chunk = plan.kb_chunk;
       p.split_compact = plan.compact;
       p.pair_parts = plan.pair_parts;
@@ -632,9 +656,13 @@ int64_t bt_prefill_partials_bytes(int32_t seqlen, int32_t q_offset, int32_t head
                                   int32_t head_dim) {
   if (seqlen < 1 || q_offset < 0 || heads < 1 || kv_heads < 1 || heads % kv_heads || head_dim < 1) return 0;
   if ((int64_t)q_offset + seqlen > INT32_MAX) return 0;
-  int64_t part_offset = 0;
-  const bt::PrefillSplitPlan plan = prefill_plan(seqlen, q_offset, heads, kv_heads, head_dim, &part_offset);
-  return plan.uses_partials() ? (int64_t)plan.part_bytes : 0;
+  const bt::PrefillSplitPlan plan = prefill8_plan(seqlen, q_offset, heads, kv_heads, head_dim);
+  if (!plan.uses_partials()) return 0;
+  // The pair kernel needs none; the query type, which decides between the
+  // kernels, is not known here.
+  const bool never = prefill_pair_faster(plan, seqlen, q_offset, heads, kv_heads, head_dim, false) &&
+                     prefill_pair_faster(plan, seqlen, q_offset, heads, kv_heads, head_dim, true);
+  return never ? 0 : (int64_t)plan.part_bytes;
 }
 
 int bt_gqa_prefill_cached(const void* q, int32_t q_dtype, const void* k, const void* v, int64_t q_stride_tok,

@@ -127,6 +127,24 @@ __host__ __device__ inline int split_items(int kb, int S, int P0, int pos, int n
   for (int c = 0; c < max_chunks; ++c) n += split_pad8(split_blocks_past(c, kb, S, P0, pos, nqb));
   return n;
 }
+// The longest-first compact grid (split_compact = 2, at most two chunks of kb
+// blocks) runs three regions of items, each ordered (query block from the
+// heaviest, subset) and padded to a multiple of 8: the first chunks of the
+// query blocks with more key blocks than the longest second chunk, the second
+// chunks, and the remaining first chunks.  longest_ahead / longest_second:
+// query blocks of the first two.
+__host__ __device__ inline int longest_ahead(int kb, int S, int P0, int pos, int nqb, int max_chunks) {
+  const int rest = (P0 + S + kKB8 - 1) / kKB8 - kb;  // blocks of the longest second chunk
+  return max_chunks > 1 && rest > 0 ? split_blocks_past(1, rest, S, P0, pos, nqb) : nqb;
+}
+__host__ __device__ inline int longest_second(int kb, int S, int P0, int pos, int nqb, int max_chunks) {
+  return max_chunks > 1 ? split_blocks_past(1, kb, S, P0, pos, nqb) : 0;
+}
+inline int longest_first_items(int kb, int S, int P0, int pos, int nqb, int max_chunks, int subsets) {
+  const int ahead = longest_ahead(kb, S, P0, pos, nqb, max_chunks);
+  return split_pad8(ahead * subsets) + split_pad8(longest_second(kb, S, P0, pos, nqb, max_chunks) * subsets) +
+         split_pad8((nqb - ahead) * subsets);
+}
 
 }  // namespace
 
@@ -170,14 +188,21 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
   constexpr int kDTiles = D / 16;      // 16-row d tiles of O^T
   constexpr int kImg = kKB8 * D * 2;   // bytes of one K or V^T tile
   constexpr int kCopies = kImg / 1024 / kWaves8;  // 1 KiB copies per wave per tile
+  // 16-byte slots of one V^T key chunk: one per row d, and in a DIRECT tile at
+  // D = 256 a free one behind every 16 rows.  There a wave writes the same row
+  // of neighbouring 8-row slices; 128 bytes apart they would meet in two of the
+  // 16 bank groups (config 4, S = 64 / 200 / 333 / 512, bf16 q: 10.6 / 14.7 /
+  // 18.7 / 19.0 -> 10.1 / 14.0 / 18.1 / 18.3 us; at D = 128 1% slower).
+  constexpr int kVRow = DIRECT && D == 256 ? D + D / 16 : D;
+  constexpr int kVImg = 8 * kVRow * 16;
 
   // Separate LDS arrays so the compiler can see that copies into one buffer
   // never alias operand reads from another; the key loop is unrolled by two so
   // every buffer choice is a constant.
   __shared__ __attribute__((aligned(1024))) unsigned char k_lds0[kImg];
   __shared__ __attribute__((aligned(1024))) unsigned char k_lds1[kImg];
-  __shared__ __attribute__((aligned(1024))) unsigned char v_lds0[kImg];
-  __shared__ __attribute__((aligned(1024))) unsigned char v_lds1[kImg];
+  __shared__ __attribute__((aligned(1024))) unsigned char v_lds0[kVImg];
+  __shared__ __attribute__((aligned(1024))) unsigned char v_lds1[kVImg];
   __shared__ uint32_t dmax[2][kWaves8];  // DIRECT: per-wave block maxima
   auto k_buf = [&](auto b) -> unsigned char* {
     if constexpr (decltype(b)::value == 0) return k_lds0; else return k_lds1;
@@ -205,7 +230,26 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
     const int ys = p.kv_heads * p.head_subs;
     int L = (int)blockIdx.x;
     bool found = false;
-    for (int c = 0; c < p.max_chunks && !found; ++c) {
+    if (p.split_compact == 2) {
+      const int ahead = longest_ahead(p.kb_chunk, S, P0, pos_per_wg, nqb, p.max_chunks);
+      const int second = longest_second(p.kb_chunk, S, P0, pos_per_wg, nqb, p.max_chunks);
+      const int end0 = split_pad8(ahead * ys), end1 = end0 + split_pad8(second * ys);
+      int items = ahead * ys, rank = 0;
+      if (L >= end1) {
+        L -= end1;
+        items = (nqb - ahead) * ys;
+        rank = ahead;
+      } else if (L >= end0) {
+        L -= end0;
+        items = second * ys;
+        split_chunk = 1;
+      }
+      if (L >= items) return;  // a padding slot (whole work-group)
+      ysub = L % ys;
+      split_qb = nqb - 1 - rank - L / ys;
+      found = true;
+    }
+    for (int c = 0; p.split_compact == 1 && c < p.max_chunks && !found; ++c) {
       const int n = split_blocks_past(c, p.kb_chunk, S, P0, pos_per_wg, nqb);
       const int np = split_pad8(n);
       if (L < np * ys) {
@@ -412,11 +456,7 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
               o[m] = to_f16(__uint_as_float((i & 1) ? (w0 & 0xffff0000u) : (w0 << 16)),
                             __uint_as_float((i & 1) ? (w1 & 0xffff0000u) : (w1 << 16)), e);
             }
-            // Row i of the slice in slot i ^ (dc & 7): a wave's lanes write the
-            // same row of neighbouring slices, 128 bytes apart, and would
-            // otherwise meet in two of the 16 bank groups (config 4, S = 64 /
-            // 333 / 500, bf16 q: 10.7 / 18.3 / 19.0 -> 10.3 / 17.8 / 18.5 us).
-            *reinterpret_cast<u32x4*>(v_buf(bsel) + (c * D + dc * 8 + (i ^ (dc & 7))) * 16) = o;
+            *reinterpret_cast<u32x4*>(v_buf(bsel) + (c * kVRow + dc * 8 + (kVRow > D ? dc >> 1 : 0) + i) * 16) = o;
           }
         } else {
           const int e = dek[b];
@@ -471,21 +511,13 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
     };
     // O^T += V^T . P^T over the 64 keys of V^T buffer b: A operand of key half kh
     // / d tile dt is chunk kh*4 + g4 of row dt*16 + i16.
-    // Row d = dt*16 + i16 lies in slot d, in a DIRECT tile with its low bits
-    // turned by those of d / 8 (see write_tiles); its offset in the 16 rows of
-    // d tile dt then depends on dt mod 4.
-    uint32_t v_row[DIRECT ? 4 : 1];
-  #pragma unroll
-    for (int m = 0; m < (DIRECT ? 4 : 1); ++m)
-      v_row[m] = (uint32_t)(DIRECT ? (i16 & 8) + ((i16 & 7) ^ (i16 >> 3) ^ (2 * m)) : i16);
     auto pv = [&](auto b, const u32x4 (&pp)[2]) {
       const unsigned char* vb_ = v_buf(b);
   #pragma unroll
       for (int kh = 0; kh < 2; ++kh) {
   #pragma unroll
         for (int dt = 0; dt < kDTiles; ++dt) {
-          const u32x4 a = *reinterpret_cast<const u32x4*>(
-              vb_ + ((kh * 4 + g4) * D + dt * 16 + v_row[DIRECT ? dt & 3 : 0]) * 16);
+          const u32x4 a = *reinterpret_cast<const u32x4*>(vb_ + ((kh * 4 + g4) * kVRow + dt * (kVRow / kDTiles) + i16) * 16);
           oacc[dt] = mfma16_f16(a, pp[kh], oacc[dt]);
         }
       }
@@ -813,8 +845,12 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
   }
 }
 
-PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv_heads, int head_dim, int num_cus) {
+PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv_heads, int head_dim, int num_cus,
+                                     bool partials) {
   PrefillSplitPlan plan;
+  // A segment's fixed cost (q rows, first tiles, last P.V, epilogue) and the
+  // combine's, in key blocks: 2 to 4 of each measured.
+  constexpr float kSegment = 3.5f, kCombine = 2.5f;
   const int pos_per_wg = kQ8 * (kWaves8 / group);
   const int nqb = (seqlen + pos_per_wg - 1) / pos_per_wg;
   plan.query_blocks = nqb;
@@ -832,12 +868,12 @@ PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv
   // stored as whole row slices) one-block chunks beat two-block ones at
   // config 4, S = 128 / 192 / 256 / 384 / 512: 13.8 / 16.6 / 17.9 / 19.3 /
   // 20.0 -> 13.2 / 14.1 / 14.8 / 16.1 / 18.6 us per call (before it, S = 128
-  // measured 24.5 against 22.3 us).  A query block has at most kMaxChunks.  A grid with a work-group per CU or more is not split
-  // (the heavy-first launch order balances it as far as it can).
+  // measured 24.5 against 22.3 us).  A query block has at most kMaxChunks.  A grid with a
+  // work-group per CU or more runs longest first (below).
   int uniform = 0;          // its chunk length (0: no uniform split)
   int longest = nkb_max;    // key blocks of the busiest work-group
   bool compact = false;
-  if ((int64_t)nqb * kv_heads < num_cus) {
+  if (partials && (int64_t)nqb * kv_heads < num_cus) {
     const int max_chunks = min(num_cus / (nqb * kv_heads), kMaxChunks);
     const int lo = (nkb_max + max_chunks - 1) / max_chunks;
     if (lo < nkb_max) {
@@ -850,7 +886,7 @@ PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv
   // 1.6 rounds of the CUs: config 4, S = 768 / 896 24.5 / 27.2 -> 22.6 / 25.9
   // us per call (288 / 392 slots); at S = 1024 (two full rounds, 512 slots)
   // 27.8 -> 38.6 us.
-  if (nkb_max > 2 && (uniform == 0 || uniform > 2) && (nkb_max + 1) / 2 <= kMaxChunks &&
+  if (partials && nkb_max > 2 && (uniform == 0 || uniform > 2) && (nkb_max + 1) / 2 <= kMaxChunks &&
       5 * (int64_t)nqb * kv_heads * ((nkb_max + 1) / 2) <= 8 * (int64_t)num_cus) {
     uniform = 2;
     longest = 2;
@@ -891,17 +927,52 @@ PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv
     const int len = n_blocks(qhi) + (r != qhi ? n_blocks(r) : 0);
     pair_longest = max(pair_longest, (len + parts - 1) / parts);
   }
-  if (uniform == 0 && pair_longest >= 2 && 3 * pair_longest < 2 * longest) {
+  if (partials && uniform == 0 && pair_longest >= 2 && 3 * pair_longest < 2 * longest) {
     plan.pair_parts = parts;
     int mc = 1;
     for (int qb = 0; qb < nqb; ++qb) mc = max(mc, pair_chunks(qb, nqb, parts, n_blocks));
     plan.max_chunks = mc;
+    plan.busiest = pair_longest + 2 * kSegment + kCombine;
   } else if (uniform > 0) {
     plan.kb_chunk = uniform;
     plan.compact = compact ? 1 : 0;
     plan.max_chunks = (nkb_max + uniform - 1) / uniform;
-  } else {
+    plan.busiest = uniform + kSegment + kCombine;
+  } else if ((int64_t)nqb * kv_heads < num_cus) {
+    plan.busiest = nkb_max + kSegment;
     return plan;
+  } else {
+    // A work-group per query block fills the CUs.  They start longest first
+    // over all subsets, the light ones filling in behind, but the kernel still
+    // lasts as long as its longest, up to 1.5 times the mean where there is
+    // little more than one round of them.  Cutting the longest at C key blocks
+    // evens that out where it pays for the further segments and the combine:
+    // H = 8, Hkv = 2, D = 256, S = 4500 bf16 / f32 q 135 / 177 -> 120 / 153 us;
+    // where the estimate gains less than 15% it measured none (H = 16, S = 3001
+    // 100 -> 110 us) and the blocks stay whole.  The order alone: Hkv = 8, D =
+    // 128, S = 1500 / 1800 55 / 67 -> 39 / 48 us.
+    int64_t total = 0;
+    for (int qb = 0; qb < nqb; ++qb) total += n_blocks(qb);
+    total *= kv_heads;
+    const float per = 1.f / num_cus;
+    // With the other CUs done, a block of the last work-groups takes 0.88 of
+    // one's time under full load.
+    const float whole = max(0.88f * (nkb_max + kSegment), (total + kSegment * nqb * kv_heads) * per);
+    int best = nkb_max;
+    float best_cost = 0.85f * whole;
+    const int first = max((nkb_max + 1) / 2, (int)(total * per));
+    for (int c = first; partials && c < nkb_max; c += 1 + nkb_max / 64) {
+      const int64_t segments = nqb + split_blocks_past(1, c, seqlen, q_offset, pos_per_wg, nqb);
+      const float cost = max(c + kSegment, 1.05f * (total + kSegment * segments * kv_heads) * per) + kCombine;
+      if (cost < best_cost) {
+        best = c;
+        best_cost = cost;
+      }
+    }
+    plan.kb_chunk = best;
+    plan.compact = 2;
+    plan.max_chunks = (nkb_max + best - 1) / best;
+    plan.busiest = best < nkb_max ? best_cost : whole;
   }
   if (plan.uses_partials()) {
     plan.part_rows = (size_t)kv_heads * nqb * plan.max_chunks * kRows8;
@@ -922,11 +993,14 @@ hipError_t launch_prefill8(const PrefillParams& p, int head_dim, hipStream_t str
   const int pos_per_wg = kQ8 * (kWaves8 / p.sub_group);
   const int nqb = (p.seqlen + pos_per_wg - 1) / pos_per_wg;
   const bool paired = p.pair_parts > 0;
-  const bool split = p.kb_chunk > 0 || (paired && p.max_chunks > 1);  // partials and the combine
+  // Partials and the combine (a heavy-first grid of whole query blocks has none).
+  const bool split = (p.kb_chunk > 0 && !(p.split_compact == 2 && p.max_chunks == 1)) || (paired && p.max_chunks > 1);
   if (paired && p.kb_chunk > 0) return hipErrorInvalidValue;
   if (split && (p.max_chunks < 1 || p.max_chunks > kMaxChunks || !p.part || !p.lse)) return hipErrorInvalidValue;
   const int ys = p.kv_heads * p.head_subs;  // grid y: (kv head, head subset)
   const dim3 grid = paired ? dim3(((nqb + 1) / 2) * p.pair_parts, ys, 1)
+                   : p.kb_chunk > 0 && p.split_compact == 2
+                       ? dim3(longest_first_items(p.kb_chunk, p.seqlen, p.q_offset, pos_per_wg, nqb, p.max_chunks, ys), 1, 1)
                    : p.kb_chunk > 0 && p.split_compact
                        ? dim3(ys * split_items(p.kb_chunk, p.seqlen, p.q_offset, pos_per_wg, nqb, p.max_chunks), 1, 1)
                        : dim3(nqb, ys, p.kb_chunk > 0 ? p.max_chunks : 1);

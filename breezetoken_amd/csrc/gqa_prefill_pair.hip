@@ -781,11 +781,15 @@ bool prefill_pair_serves(int group, int head_dim) {
   return group == 1 || group == 2 || group == 4 || group == 8;
 }
 
-// Work-groups of the bf16-q launch (two q-tiles per wave); the f32-q launch
-// (one q-tile per wave, hi + lo q) has twice as many, each with half the work.
-int prefill_pair_grid(int seqlen, int group, int kv_heads) {
-  const PairShape sh = pair_shape(group, 2);
+// The f32-q launch (one q-tile per wave, hi + lo q) has twice as many
+// work-groups as the bf16-q one (two q-tiles per wave), each with half the
+// work.  Together a pair's two query blocks take the same steps whatever
+// blocks they are (see pair_group).
+int prefill_pair_grid(int seqlen, int q_offset, int group, int kv_heads, bool q_f32, int* steps) {
+  const PairShape sh = pair_shape(group, q_f32 ? 1 : 2);
   const int nqb = (seqlen + sh.pos - 1) / sh.pos;
+  auto n_units = [&](int blk) { return (q_offset + min(seqlen, (blk + 1) * sh.pos) + kUnit - 1) / kUnit; };
+  *steps = (n_units(nqb - 1) + (nqb > 1 ? n_units(0) : 0)) / 2 + 1;
   return ((nqb + 1) / 2) * kv_heads * sh.nsub;
 }
 
