@@ -20,9 +20,11 @@
 //    h and 2*GMAX-1-h), so Q.K^T keeps ~16 mantissa bits although the MFMA takes
 //    bf16; the two halves are summed with one DPP mirror.  P is split the same
 //    way for the P.V product;
-//  * S^T = K . Q^T puts the K tile in the A operand, so K rows go straight from
-//    HBM into registers with 16-byte buffer loads (64 contiguous bytes per token
-//    per instruction); loads past the valid length return zero (buffer bounds);
+//  * S^T = K . Q^T puts the K tile in the A operand.  K is read in whole token
+//    rows and turned into that layout through the wave's LDS tile; calls with few
+//    tiles per wave read it straight into registers in the operand layout instead
+//    (64 contiguous bytes per token per instruction).  Loads are 16-byte buffer
+//    loads; those past the valid length return zero (buffer bounds);
 //  * V is staged through an XOR-swizzled LDS tile per wave and read back with
 //    ds_read_b64_tr_b16, which yields the V^T operand of O^T = V^T . P^T without
 //    any shuffle; the lane that owns score column n for tokens t also owns the
@@ -109,17 +111,25 @@ enum DecodeMode : int {
 // instead of leaving most waves of 128 work-groups idle, and the splits past
 // ns_eff write lse = -inf at once.
 //
-// Per tile and wave, K (16 tokens x D) and V land in registers; K feeds the
-// MFMA directly, V is staged through the wave's XOR-swizzled LDS tile and read
-// back transposed.  A wave requests its next V as soon as the current V is in
-// LDS, and its next K as soon as Q.K^T has consumed the current one -- except
-// after the first tile, where the next K goes out with the next V.  A wave's
-// first tile is requested after its slice of Q^T is built (wave 0's, at entry).
+// Per tile and wave, K (16 tokens x D) and V land in registers; each is staged
+// through the wave's XOR-swizzled LDS tile in turn (K only with ROWS: without it
+// the registers feed the MFMA) and V is read back transposed.  A wave requests
+// its next V as soon as the current V is in LDS, and its next K as soon as its
+// registers are free -- except after the first tile, where the next K goes out
+// with the next V.  A wave's first tile is requested after its slice of Q^T is
+// built (wave 0's, at entry).
 //
 // ONE: every sequence has one split, whose merged rows are the results: they go
 // to p.out and no combine follows.  Its own instantiation, so the split kernel
 // keeps its arguments and registers.
-template <int GMAX, int D, int W, int MODE, bool QBF16, bool ONE>
+//
+// ROWS: K is read in whole rows and brought into the operand layout through the
+// wave's LDS tile, instead of straight into registers in 64-byte pieces of 16
+// rows.  The HBM serves whole rows faster (64 MiB by the split kernel's groups:
+// 72% of its peak against 66%), and the extra pass hides behind the other
+// waves' tiles; with a tile per wave it is only latency (~0.1 us).  Which launch
+// takes which form: see kRowsMinSlots.
+template <int GMAX, int D, int W, int MODE, bool QBF16, bool ONE, bool ROWS>
 __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplitParams p) {
   constexpr int kThreads = W * 64;
   constexpr int kSteps = D / 32;            // K-dimension steps of Q.K^T
@@ -227,7 +237,11 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
   }
 
   // ---- K/V addressing -------------------------------------------------------
-  // K: lane (col, kg) holds token col's 16 bytes kg of each 64-byte d-step.
+  // K, operand form: lane (col, kg) holds token col's 16 bytes kg of each
+  // 64-byte d-step, which the MFMA takes as they are.
+  // K, row form: load j fetches whole token rows as V's does; chunk c of token
+  // row r goes to slot c ^ (r & 15) of the wave's LDS tile, so that the operand
+  // reads of 16 rows fall on 16 bank groups.
   // V: load j of a tile fills LDS bytes [1024 j, +1024) of the wave's tile;
   // lane l fetches the chunk that belongs in its slot (the swizzle is applied
   // on the source side).
@@ -239,6 +253,11 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
     return (uint32_t)(lane / kSlots) * row_bytes + (uint32_t)((lane % kSlots) ^ swz(r, kSlots)) * 16;
   };
 
+  auto kvoff = [&](int j) -> uint32_t {
+    const int r = j * kRowsPerLoad + lane / kSlots;
+    return (uint32_t)(lane / kSlots) * row_bytes + (uint32_t)((lane % kSlots) ^ (r & 15 & (kSlots - 1))) * 16;
+  };
+
   // Speculative path (device position, single sequence): the split's first
   // tile is tile s whatever ns_eff turns out to be, so wave 0 fetches it inside
   // the capacity bound before the position is known; rows past the valid
@@ -248,12 +267,16 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
   __amdgpu_buffer_rsrc_t krs = make_rsrc(p.k + head_off0, (uint32_t)p.seqlen * row_bytes);
   __amdgpu_buffer_rsrc_t vrs = make_rsrc(p.v + head_off0, (uint32_t)p.seqlen * row_bytes);
 
+  static_assert(kSteps == kVLoads, "a K tile is as many loads in either form");
   u32x4 kr[kSteps];
   u32x4 vr[kVLoads];
   auto issue_k = [&](int tile) {
     const uint32_t so = (uint32_t)tile * 16 * row_bytes;
 #pragma unroll
-    for (int st = 0; st < kSteps; ++st) kr[st] = buf_load16(krs, koff + st * 64, so);
+    for (int st = 0; st < kSteps; ++st) {
+      if constexpr (ROWS) kr[st] = buf_load16(krs, kvoff(st), so + (uint32_t)(st * kRowsPerLoad) * row_bytes);
+      else kr[st] = buf_load16(krs, koff + st * 64, so);
+    }
   };
   auto issue_v = [&](int tile) {
     const uint32_t so = (uint32_t)tile * 16 * row_bytes;
@@ -358,18 +381,39 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
     u32x4 qop[kSteps];
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) qop[st] = qlds[st * 64 + lane];
+    if constexpr (ROWS) {
 #pragma unroll
-    for (int st = 0; st < kSteps; ++st) sacc = mfma16(as_bf16x8(kr[st]), as_bf16x8(qop[st]), sacc);
-    // The next K goes out here, except after the first tile: there it waits
-    // for the V staging, which keeps the compiler's waits at the first Q.K^T
-    // exact (each MFMA waits for its own K load) without the next requests
-    // joining the queue while the first V is still arriving (4k -0.2 us,
-    // C3 32k -0.18 us, 32k -0.08 us; issued late in every step, 131k +0.9 us).
-    if (more && !first) issue_k(tile + tstride);
-    // Stage V in this wave's swizzled LDS tile (same-wave LDS ops stay
-    // ordered) and request the next V.  Rows past the valid length are zeros
-    // (buffer range), except in a speculative tile read inside the capacity:
-    // there they are zeroed here, since p = 0 on them but 0 * NaN is not 0.
+      for (int j = 0; j < kSteps; ++j)
+        *reinterpret_cast<BT_LDS u32x4*>((BT_LDS unsigned char*)vtile + j * 1024 + lane * 16) = kr[j];
+      if (more && !first) issue_k(tile + tstride);
+      u32x4 kop[kSteps];
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st)
+        kop[st] = *reinterpret_cast<const BT_LDS u32x4*>((BT_LDS unsigned char*)vtile + col * kRowBytes +
+                                                         (((st * 4 + kg) ^ (col & (kSlots - 1))) * 16));
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st) sacc = mfma16(as_bf16x8(kop[st]), as_bf16x8(qop[st]), sacc);
+      // The scores leave the matrix unit through this fence.  An MFMA's result
+      // may be read 8 wait states after it; hipcc 7.2 counts them over the code
+      // in a row, but where the last MFMA was followed by a branch it put 2 on
+      // the path that takes it, and D = 64 read stale scores.  The nop is tied
+      // to the registers, so nothing that reads them moves ahead of it.
+      asm volatile("s_nop 7" : "+v"(sacc));
+    } else {
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st) sacc = mfma16(as_bf16x8(kr[st]), as_bf16x8(qop[st]), sacc);
+      // The next K goes out here, except after the first tile: there it waits
+      // for the V staging, which keeps the compiler's waits at the first Q.K^T
+      // exact (each MFMA waits for its own K load) without the next requests
+      // joining the queue while the first V is still arriving (4k -0.2 us,
+      // C3 32k -0.18 us, 32k -0.08 us; issued late in every step, 131k +0.9 us).
+      if (more && !first) issue_k(tile + tstride);
+    }
+    // Stage V in this wave's swizzled LDS tile (behind K's operand reads:
+    // same-wave LDS ops stay ordered) and request the next V.  Rows past the
+    // valid length are zeros (buffer range), except in a speculative tile read
+    // inside the capacity: there they are zeroed here, since p = 0 on them but
+    // 0 * NaN is not 0.
     const bool spec_tail = kSpec && first && spec_loaded && tile * 16 + 16 > valid;
 #pragma unroll
     for (int j = 0; j < kVLoads; ++j) {
@@ -643,18 +687,36 @@ __global__ __launch_bounds__(64) void gqa_decode_combine_kernel(CombineParams p)
   }
 }
 
+// Whether a launch reads K in whole rows (ROWS).  Always, except by device
+// position at D = 256 where waves get too few tiles for the better stream to pay
+// for the LDS pass: groups of up to 4 heads, one split, caches under 16,384
+// slots.  us per call, pieces -> rows: H = 16, Hkv = 2, D = 256 at 32k / 131k
+// 17.85 / 49.9 -> 16.9 / 48.2; H = 32, Hkv = 8, D = 128 at 4k / 32k 8.9 / 28.6 ->
+// 8.6 / 25.5; ragged 32 x 256 .. 32,768 tokens, D = 256, 83.7 -> 77.8, 24 x 256
+// .. 4,000, D = 128, 39.7 -> 36.0.  H = 8, Hkv = 2, D = 256 by position gains 1%
+// at 32k (15.9 -> 15.7) and loses 2% at 1k and 4k (6.65 -> 6.75, 7.40 -> 7.54).
+constexpr int kRowsMinSlots = 16384;
+
 template <int GMAX, int D, int MODE, bool QBF16>
 static hipError_t launch_split_t(const DecodeSplitParams& p, int grid_x, int batch, hipStream_t stream) {
   const dim3 grid(grid_x * p.kv_heads, 1, batch), block(kDecodeWaves * 64);
+  auto launch = [&](auto one, auto rows) {
+    hipLaunchKernelGGL((gqa_decode_split_kernel<GMAX, D, kDecodeWaves, MODE, QBF16, decltype(one)::value != 0,
+                                                decltype(rows)::value != 0>),
+                       grid, block, 0, stream, p);
+    return hipGetLastError();
+  };
+  constexpr bool kPieces = MODE == kModePos && D == 256;
   if constexpr (MODE != kModeRagged) {
     if (p.out) {
       if (p.num_split != 1 || grid_x != 1) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((gqa_decode_split_kernel<GMAX, D, kDecodeWaves, MODE, QBF16, true>), grid, block, 0, stream, p);
-      return hipGetLastError();
+      return launch(IntConst<1>{}, IntConst<!kPieces>{});
     }
   }
-  hipLaunchKernelGGL((gqa_decode_split_kernel<GMAX, D, kDecodeWaves, MODE, QBF16, false>), grid, block, 0, stream, p);
-  return hipGetLastError();
+  if constexpr (kPieces && GMAX > 4) {
+    if (p.seqlen >= kRowsMinSlots) return launch(IntConst<0>{}, IntConst<1>{});
+  }
+  return launch(IntConst<0>{}, IntConst<!kPieces>{});
 }
 
 template <int GMAX, int D>
