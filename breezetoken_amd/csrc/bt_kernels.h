@@ -185,32 +185,71 @@ struct GemvParams {
   float* y;              // (N,) f32
 };
 
-// Launch shape of the matvec: VEC columns per lane (tile = 64*VEC columns)
-// and the number of K shares.  A wide matrix (>= 256 tiles of 512 columns,
-// e.g. the vocabulary head) is not split: every CU already streams whole
-// columns.  Otherwise K is split so that about 512 work-groups stream W with
-// at least 64 rows per share (measured on MI355X against 256/1024/2048/4096
-// groups and 16/32/128 rows).
+// Launch shape of the matvec, for one of two kernels (gemv.hip).
+//
+// vec > 0: the column kernel, VEC columns per lane (tile = 64*VEC columns) and
+// `splits` shares of K.  A wide matrix (>= 256 tiles of 512 columns, e.g. the
+// vocabulary head) is not split: every CU already streams whole columns.
+// Otherwise about 512 work-groups stream W with at least 64 rows per share.
+// lanes > 0: the strip kernel, `lanes` lanes across a strip of 8 * lanes
+// columns.  It takes, per the rates beside it,
+//  * K of 256..1536 without a split, where strips fill the chip: strips of 32
+//    columns for N of 3072 per 512 rows up to 8192 (256 work-groups: 9216 takes a
+//    second round, 1024 x 9216 9.8 us against 8.2), of 64 from there to 16,384
+//    (the same), of 128 from there to 65,536 (1024 x 100,000 45.3 us against
+//    42.4); past K = 1024 the last two begin at 12,288 and 24,576 columns;
+//  * else K > 2048, or K > 1024 and N >= 4096, up to N = 32,768, in strips of 128
+//    columns and shares of one pass (256 rows), at most 1024 work-groups.  Where
+//    that makes 257..512 of them, a second round that is not full, shares are 512
+//    rows if then all run at once.
+// Two pitches stay with the column kernel: rows that do not begin on a line, where
+// strips share lines, for N and K under 4096 (2560 x 1000 6.57 us against 6.45);
+// and rows of 4 KB from K = 6144, whose strips land on few memory channels (12,288
+// x 2048 13.2 us against 12.1; 8192 x 2048 would gain, 11.9 -> 9.4).
 constexpr int kGemvTargetGroups = 512;
 constexpr int kGemvMinRows = 64;
-inline void gemv_shape(int K, int N, int* vec, int* splits, int* tiles) {
+struct GemvShape {
+  int vec, lanes, splits, tiles;
+};
+inline GemvShape gemv_shape(int K, int N) {
+  GemvShape g{};
   const int tiles8 = (N + 511) / 512;
-  *vec = tiles8 >= 8 ? 8 : 4;
-  *tiles = (N + 64 * *vec - 1) / (64 * *vec);
-  if (tiles8 >= 256) {
-    *splits = 1;
-    return;
+  if (tiles8 < 256) {
+    const bool narrow = N >= 3072 * ((K + 511) / 512) && N <= 8192;
+    const bool middle = N > (K <= 1024 ? 8192 : 12287) && N <= 16384;
+    const bool wide = N > (K <= 1024 ? 16384 : 24575) && N <= 65536;
+    if (K >= 256 && K <= 1536 && (narrow || middle || wide)) {
+      g.lanes = narrow ? 4 : middle ? 8 : 16;
+      g.tiles = (N + 8 * g.lanes - 1) / (8 * g.lanes);
+      g.splits = 1;
+      return g;
+    }
+    const bool lines = N % 128 == 0 || N >= 4096 || K >= 4096;
+    const bool channels = N != 2048 || K < 6144;
+    if ((K > 2048 || (K > 1024 && N >= 4096)) && lines && channels && N <= 32768) {
+      g.lanes = 16;
+      g.tiles = (N + 127) / 128;
+      const int one = (K + 255) / 256, two = (K + 511) / 512, cap = 1024 / g.tiles;
+      const int64_t groups = (int64_t)g.tiles * one;
+      const int sk = groups > 256 && groups <= 512 && g.tiles * two <= 256 ? two : one;
+      g.splits = sk < cap ? sk : cap;
+      return g;
+    }
   }
-  const int sk = (kGemvTargetGroups + *tiles - 1) / *tiles;
+  g.vec = tiles8 >= 8 ? 8 : 4;
+  g.tiles = (N + 64 * g.vec - 1) / (64 * g.vec);
+  g.splits = 1;
+  if (tiles8 >= 256) return g;
+  const int sk = (kGemvTargetGroups + g.tiles - 1) / g.tiles;
   const int cap = K / kGemvMinRows > 1 ? K / kGemvMinRows : 1;
-  *splits = sk < 1 ? 1 : (sk > cap ? cap : sk);
+  g.splits = sk < 1 ? 1 : (sk > cap ? cap : sk);
+  return g;
 }
 
 // Workspace of the split-K matvec: the partial rows.
 inline size_t gemv_workspace_bytes(int K, int N) {
-  int vec, sk, tiles;
-  gemv_shape(K, N, &vec, &sk, &tiles);
-  return sk == 1 ? 0 : (size_t)sk * N * 4;
+  const GemvShape g = gemv_shape(K, N);
+  return g.splits == 1 ? 0 : (size_t)g.splits * N * 4;
 }
 
 // Keys per block of the prefill key loop, and the size of the transposed,
@@ -286,6 +325,6 @@ hipError_t launch_prefill8(const PrefillParams& p, int head_dim, hipStream_t str
 hipError_t launch_row_norm_rope(const RowPrepParams& p, int head_dim, hipStream_t stream);
 hipError_t launch_attn_prep(const RowPrepParams& p, int head_dim, hipStream_t stream);
 hipError_t launch_gdn_decode(const GdnParams& p, int dim, hipStream_t stream);
-hipError_t launch_gemv(const GemvParams& p, int vec, hipStream_t stream);
+hipError_t launch_gemv(const GemvParams& p, const GemvShape& shape, hipStream_t stream);
 
 }  // namespace bt

@@ -776,20 +776,19 @@ int bt_gemv_bf16(const float* x, const void* w, int64_t ldw, int32_t K, int32_t 
   if (!x || !w || !y || K < 1 || N < 1 || ldw < N) return BT_EINVAL;
   if (N % 8 || ldw % 8 || !aligned16(w)) return BT_EINVAL;
   if ((int64_t)K * ldw * 2 > (int64_t)INT32_MAX) return BT_ENOTSUP;
-  int vec, sk, tiles;
-  bt::gemv_shape(K, N, &vec, &sk, &tiles);
+  const bt::GemvShape shape = bt::gemv_shape(K, N);
   const int64_t need = (int64_t)bt::gemv_workspace_bytes(K, N);
-  if (sk > 1 && (!workspace || !aligned16(workspace) || workspace_bytes < need)) return BT_ENOSPC;
+  if (shape.splits > 1 && (!workspace || !aligned16(workspace) || workspace_bytes < need)) return BT_ENOSPC;
   bt::GemvParams p{};
   p.x = x;
   p.w = static_cast<const uint16_t*>(w);
   p.ldw = ldw;
   p.K = K;
   p.N = N;
-  p.splits = sk;
+  p.splits = shape.splits;
   p.partial = static_cast<float*>(workspace);
   p.y = y;
-  return hip_rc(bt::launch_gemv(p, vec, (hipStream_t)stream));
+  return hip_rc(bt::launch_gemv(p, shape, (hipStream_t)stream));
 }
 
 }  // extern "C"
