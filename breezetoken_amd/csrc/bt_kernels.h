@@ -124,6 +124,7 @@ struct PrefillSplitPlan {
   size_t part_rows = 0;    // kv_heads x query_blocks x max_chunks x rows per work-group
   size_t part_bytes = 0;   // part_rows x (head_dim f32 partials + 1 f32 LSE)
   float busiest = 0;       // estimate: key blocks of the busiest CU, its fixed costs among them
+  bool idle = false;       // a work-group per query block, fewer of them than CUs
   bool active() const { return kb_chunk > 0 || pair_parts > 0; }
   bool uses_partials() const { return active() && max_chunks > 1; }
 };

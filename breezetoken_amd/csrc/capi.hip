@@ -132,30 +132,60 @@ bt::PrefillSplitPlan prefill8_plan(int32_t seqlen, int32_t q_offset, int32_t hea
 // time is a whole number of rounds, and a grid just past one costs two: at S =
 // 4500 it took 257 us against 187 (H = 16, Hkv = 2, D = 256, bf16 q), 182
 // against 117 (D = 128).  Within one round it is the faster one once its steps
-// outweigh its start and final merge: bf16 q, H = 8, S = 6000 / 8192 180 /
-// 255 against 181 / 283 us; f32 q, whose pair work-groups are half as large,
-// H = 8, S = 3001 82 against 100, H = 16, S = 1500 53 against 67 us.  The
-// constants (us per call, per step, per 64-key block) fit these and S = 1024
-// .. 8192 at four shapes to about 10%.
+// outweigh its start and final merge: H = 8, Hkv = 2, D = 256, bf16 q, S = 7000
+// 209 against 217 us; f32 q, whose pair work-groups are half as large, S =
+// 1024 41 against 51 us, 3001 82 against 120 us (no partials).  A grid that
+// leaves CUs idle lasts as long as its longest work-group, whose blocks take
+// less than under full load, and starts sooner: bf16 q, S = 1024 / 2048 / 3001
+// 41 / 69 / 95 us against the pair kernel's 53 / 80 / 104.
+// The rates (us) are fits to S = 130 .. 16,384 at four shapes for each head
+// dimension and q type, medians over seven rounds in turn; over those 900 choices
+// the kernel taken is the faster one or within 1% of it, but for three (4%).
+struct PrefillRates {
+  double pair_start, pair_step;    // pair kernel: per call, per step of 32 keys
+  double two_start, two_block;     // two-wave kernel: per call, per 64-key block of the busiest CU
+  double idle_start, idle_factor;  // the same where CUs stay idle: per call, of two_block
+  double paired_factor;            // a block of the paired split, of two_block
+};
 bool prefill_pair_faster(const bt::PrefillSplitPlan& plan, int32_t seqlen, int32_t q_offset, int32_t heads,
                          int32_t kv_heads, int32_t head_dim, bool q_f32) {
   const int group = heads / kv_heads;
   if (!bt::prefill_pair_serves(group, head_dim)) return false;
   const bool wide = head_dim == 256;
+  const PrefillRates r = wide ? (q_f32 ? PrefillRates{17.0, 1.36, 10.0, 2.55, 6.0, 0.88, 1.05}
+                                       : PrefillRates{23.0, 1.68, 11.0, 2.0, 5.0, 0.88, 1.12})
+                              : (q_f32 ? PrefillRates{12.5, 0.89, 10.0, 1.4, 5.0, 0.97, 1.1}
+                                       : PrefillRates{15.0, 1.17, 10.0, 1.18, 5.0, 1.0, 1.1});
   const int64_t cus = device_cus();
   int steps = 0;
   const int64_t groups = bt::prefill_pair_grid(seqlen, q_offset, group, kv_heads, q_f32, &steps);
   double rounds = (double)((groups + cus - 1) / cus);
-  // At D = 128 two f32-q work-groups fit a CU and take 1.4 times one's time;
+  // At D = 128 two f32-q work-groups fit a CU and take 1.56 times one's time;
   // half-filled rounds of two pass as such.
-  if (!wide && q_f32 && groups > cus) rounds = 1.4 * std::max(1.0, 0.5 * (double)((groups + cus - 1) / cus));
-  const double base = wide ? (q_f32 ? 17.0 : 18.0) : (q_f32 ? 11.0 : 13.0);
-  const double step = wide ? (q_f32 ? 1.42 : 1.7) : (q_f32 ? 0.97 : 1.2);
-  const double block = wide ? (q_f32 ? 2.55 : 2.05) : (q_f32 ? 1.36 : 1.14);
+  if (!wide && q_f32 && groups > cus) rounds = 1.56 * std::max(1.0, 0.5 * (double)((groups + cus - 1) / cus));
+  const double pair = r.pair_start + rounds * steps * r.pair_step;
   // Short prompts whose work-groups convert their own blocks have no pre-pass.
   const int64_t longest = ((int64_t)q_offset + seqlen + bt::kPrefillKeyBlock - 1) / bt::kPrefillKeyBlock;
-  const double base8 = (plan.kb_chunk > 0 ? plan.kb_chunk : longest) <= 2 ? 4.0 : 10.0;
-  return base + rounds * steps * step < 0.95 * (base8 + plan.busiest * block);
+  const double start = (plan.kb_chunk > 0 ? plan.kb_chunk : longest) <= 2 ? 4.0 : r.two_start;
+  double two = start + plan.busiest * r.two_block * (plan.pair_parts > 0 ? r.paired_factor : 1.0);
+  if (plan.idle) two = r.idle_start + plan.busiest * r.two_block * r.idle_factor;
+  // Plans of whole query blocks, or with the longest cut, are fitted to 3%, the others to 10%.
+  const bool close = plan.pair_parts == 0 && (plan.compact == 2 || plan.kb_chunk == 0);
+  return pair < (close ? 0.99 : 0.95) * two;
+}
+
+// What bt_gqa_prefill and bt_gqa_prefill_cached run for a call whose partials
+// may take `partials_bytes`.
+struct PrefillChoice {
+  bool pair;
+  bt::PrefillSplitPlan plan;  // of the two-wave kernel
+};
+PrefillChoice prefill_choice(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads, int32_t head_dim,
+                             bool q_f32, int64_t partials_bytes) {
+  bt::PrefillSplitPlan plan = prefill8_plan(seqlen, q_offset, heads, kv_heads, head_dim);
+  if (plan.uses_partials() && partials_bytes < (int64_t)plan.part_bytes)
+    plan = prefill8_plan(seqlen, q_offset, heads, kv_heads, head_dim, false);
+  return {prefill_pair_faster(plan, seqlen, q_offset, heads, kv_heads, head_dim, q_f32), plan};
 }
 
 }  // namespace
@@ -605,10 +635,10 @@ static int prefill_run(const void* q, int32_t q_dtype, const void* k, const void
   p.img_first = img_first_key / bt::kPrefillKeyBlock;
   p.q_f32 = q_dtype == BT_DTYPE_F32 ? 1 : 0;
   p.keep_images = keep_images ? 1 : 0;
-  bt::PrefillSplitPlan plan = prefill8_plan(seqlen, q_offset, heads, kv_heads, head_dim);
-  if (plan.uses_partials() && !(partials && partials_bytes >= (int64_t)plan.part_bytes))
-    plan = prefill8_plan(seqlen, q_offset, heads, kv_heads, head_dim, false);
-  if (prefill_pair_faster(plan, seqlen, q_offset, heads, kv_heads, head_dim, p.q_f32 != 0))
+  const PrefillChoice choice = prefill_choice(seqlen, q_offset, heads, kv_heads, head_dim, p.q_f32 != 0,
+                                              partials ? partials_bytes : 0);
+  const bt::PrefillSplitPlan& plan = choice.plan;
+  if (choice.pair)
     return hip_rc(bt::launch_prefill_pair(p, head_dim, (hipStream_t)stream));
   // Every other shape runs two waves per SIMD (groups of 3, 5, 6, 7 as
   // subsets of 1 or 2 heads).  When one work-group per query block would
@@ -663,6 +693,22 @@ int64_t bt_prefill_partials_bytes(int32_t seqlen, int32_t q_offset, int32_t head
   const bool never = prefill_pair_faster(plan, seqlen, q_offset, heads, kv_heads, head_dim, false) &&
                      prefill_pair_faster(plan, seqlen, q_offset, heads, kv_heads, head_dim, true);
   return never ? 0 : (int64_t)plan.part_bytes;
+}
+
+int bt_prefill_plan(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads, int32_t head_dim,
+                    int32_t q_dtype, int64_t partials_bytes, int32_t* plan) {
+  if (!plan || seqlen < 1 || q_offset < 0 || heads < 1 || kv_heads < 1 || heads % kv_heads) return BT_EINVAL;
+  if ((int64_t)q_offset + seqlen > INT32_MAX) return BT_EINVAL;
+  if (q_dtype != BT_DTYPE_F32 && q_dtype != BT_DTYPE_BF16) return BT_EINVAL;
+  if (!bt::prefill8_serves(heads / kv_heads, head_dim)) return BT_ENOTSUP;
+  const PrefillChoice c =
+      prefill_choice(seqlen, q_offset, heads, kv_heads, head_dim, q_dtype == BT_DTYPE_F32, partials_bytes);
+  plan[0] = c.pair ? 1 : 0;
+  plan[1] = c.pair ? 0 : c.plan.kb_chunk;
+  plan[2] = c.pair ? 1 : c.plan.max_chunks;
+  plan[3] = c.pair ? 0 : c.plan.compact;
+  plan[4] = c.pair ? 0 : c.plan.pair_parts;
+  return BT_OK;
 }
 
 int bt_gqa_prefill_cached(const void* q, int32_t q_dtype, const void* k, const void* v, int64_t q_stride_tok,

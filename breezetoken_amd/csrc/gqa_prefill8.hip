@@ -940,6 +940,7 @@ PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv
     plan.busiest = uniform + kSegment + kCombine;
   } else if ((int64_t)nqb * kv_heads < num_cus) {
     plan.busiest = nkb_max + kSegment;
+    plan.idle = true;
     return plan;
   } else {
     // A work-group per query block fills the CUs.  They start longest first

@@ -235,6 +235,17 @@ int bt_gqa_prefill(const void* q, int32_t q_dtype, const void* k, const void* v,
 int64_t bt_prefill_partials_bytes(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads,
                                   int32_t head_dim);
 
+/* How bt_gqa_prefill runs a call of this shape on the current device when its
+ * partials may take partials_bytes, without running it: plan[0] 1 for the pair
+ * kernel (two query blocks per work-group; the rest is then 0, with one chunk),
+ * 0 for the two-waves-per-SIMD kernel; plan[1] the key blocks of 64 per chunk
+ * (0: no uniform chunks); plan[2] the most chunks a query block has; plan[3] the
+ * grid's order (0 query blocks by subset, 1 chunk by chunk, 2 longest first over
+ * all subsets); plan[4] the work-groups per pair of query blocks (0: no paired
+ * split).  No reference counterpart. */
+int bt_prefill_plan(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads, int32_t head_dim,
+                    int32_t q_dtype, int64_t partials_bytes, int32_t* plan);
+
 /* bt_gqa_prefill for chunked prefill over one cache, with the K / V^T images
  * kept across calls instead of rebuilt from the whole prefix each time (the
  * chunk loop of Qwen36MoE._attn_batch, breezetoken/model/qwen36_moe.py:

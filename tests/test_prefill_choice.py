@@ -1,0 +1,60 @@
+"""Which prefill kernel a call takes, by the library's estimate of both (bt_prefill_plan;
+256 CUs where no GPU is present).  The choices asserted are the measured faster ones."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+from breezetoken_amd import _lib
+
+ALL = 1 << 40  # room for any partials
+
+
+def prefill_plan(steps, heads, kv, dim, q_f32, room=ALL, q_offset=0):
+    out = (ctypes.c_int32 * 5)()
+    _lib.check("bt_prefill_plan", _lib.lib().bt_prefill_plan(
+        steps, q_offset, heads, kv, dim, _lib.BT_DTYPE_F32 if q_f32 else _lib.BT_DTYPE_BF16, room,
+        ctypes.addressof(out)))
+    return dict(zip(("pair", "chunk", "chunks", "order", "parts"), out))
+
+
+# us, pair kernel against two waves per SIMD
+@pytest.mark.parametrize("steps,heads,kv,dim,q_f32,pair", [
+    (256, 8, 2, 256, True, False),     # 24.1 / 23.2
+    (256, 16, 2, 128, True, False),    # 16.6 / 15.5
+    (1024, 8, 2, 256, True, True),     # 41.0 / 50.9
+    (1024, 8, 2, 256, False, False),   # 52.6 / 40.7
+    (2048, 8, 2, 256, False, False),   # 80.3 / 68.7
+    (3001, 8, 2, 256, False, False),   # 104 / 95
+    (3001, 8, 2, 256, True, True),     # 82 / 120
+    (1500, 16, 2, 256, False, False),  # 66.7 / 55.9
+    (2048, 4, 4, 256, False, False),   # 83.5 / 71.1
+])
+def test_calls_without_partials_take_the_faster_kernel(steps, heads, kv, dim, q_f32, pair):
+    """Grids that leave CUs idle, where the two-wave kernel's blocks are faster than under load."""
+    got = prefill_plan(steps, heads, kv, dim, q_f32, room=0)
+    assert got["pair"] == pair and got["chunks"] == 1 and got["parts"] == 0
+
+
+@pytest.mark.parametrize("steps,heads,kv,dim,q_f32,pair", [
+    (8192, 8, 2, 256, False, True),    # 254 / 277
+    (6000, 8, 2, 256, True, False),    # 260 / 235
+    (8192, 16, 2, 128, False, True),   # 312 / 314
+    (16384, 16, 2, 128, True, True),   # 1397 / 1443
+    (7000, 32, 8, 128, True, True),    # 547 / 565
+    (768, 32, 8, 128, False, False),   # 33.4 / 31.0
+    (4500, 16, 2, 256, True, False),   # 306 / 242
+])
+def test_calls_with_partials_take_the_faster_kernel(steps, heads, kv, dim, q_f32, pair):
+    assert prefill_plan(steps, heads, kv, dim, q_f32)["pair"] == pair
+
+
+def test_plan_refuses_what_the_call_refuses():
+    lib, out = _lib.lib(), (ctypes.c_int32 * 5)()
+    assert lib.bt_prefill_plan(8, 0, 8, 2, 64, _lib.BT_DTYPE_F32, 0, ctypes.addressof(out)) == _lib.BT_ENOTSUP
+    assert lib.bt_prefill_plan(0, 0, 8, 2, 256, _lib.BT_DTYPE_F32, 0, ctypes.addressof(out)) == _lib.BT_EINVAL
+    assert lib.bt_prefill_plan(8, 0, 9, 2, 256, _lib.BT_DTYPE_F32, 0, ctypes.addressof(out)) == _lib.BT_EINVAL
+    assert lib.bt_prefill_plan(8, 0, 8, 2, 256, 7, 0, ctypes.addressof(out)) == _lib.BT_EINVAL
+    assert lib.bt_prefill_plan(8, 0, 8, 2, 256, _lib.BT_DTYPE_F32, 0, None) == _lib.BT_EINVAL
