@@ -51,6 +51,22 @@ def test_calls_with_partials_take_the_faster_kernel(steps, heads, kv, dim, q_f32
     assert prefill_plan(steps, heads, kv, dim, q_f32)["pair"] == pair
 
 
+# us, query blocks by subset (0) against longest first over all subsets (2)
+@pytest.mark.parametrize("steps,heads,kv,dim,q_f32,order", [
+    (3001, 16, 2, 256, True, 0),   # 126.7 / 128.1
+    (2600, 16, 2, 256, True, 0),   # 111.1 / 111.9
+    (6000, 8, 2, 256, True, 0),    # 235.3 / 239.2
+    (3504, 16, 2, 256, True, 0),   # the last with 219 query blocks
+    (3505, 16, 2, 256, True, 2),
+    (3584, 16, 2, 256, True, 2),   # 161.5 / 155.0
+    (1500, 32, 8, 128, False, 2),  # 56.6 / 39.3, eight subsets
+    (12000, 4, 4, 256, True, 2),   # 555 / 461, four
+])
+def test_order_of_whole_query_blocks(steps, heads, kv, dim, q_f32, order):
+    got = prefill_plan(steps, heads, kv, dim, q_f32, room=0)
+    assert (got["pair"], got["chunks"], got["order"]) == (0, 1, order)
+
+
 def test_plan_refuses_what_the_call_refuses():
     lib, out = _lib.lib(), (ctypes.c_int32 * 5)()
     assert lib.bt_prefill_plan(8, 0, 8, 2, 64, _lib.BT_DTYPE_F32, 0, ctypes.addressof(out)) == _lib.BT_ENOTSUP
