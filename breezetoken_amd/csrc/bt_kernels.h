@@ -109,8 +109,9 @@ struct PrefillParams {
   // by more than one range writes partials for prefill_combine_kernel.
   int32_t pair_parts;
   int32_t max_chunks;  // chunks of the longest query block (grid z of the uniform split)
-  float* part;         // (kv_heads, query blocks, max_chunks, 128 rows, D) f32
-  float* lse;          // (kv_heads, query blocks, max_chunks, 128 rows) f32
+  int32_t part_blocks; // query blocks per subset with room for partials: the last ones
+  float* part;         // (subsets, part_blocks, max_chunks, 128 rows, D) f32
+  float* lse;          // (subsets, part_blocks, max_chunks, 128 rows) f32
 };
 
 // Split-key plan of the two-waves-per-SIMD prefill: used when one work-group
@@ -121,7 +122,8 @@ struct PrefillSplitPlan {
   int32_t pair_parts = 0;  // 0: no paired split
   int32_t max_chunks = 1;
   int32_t query_blocks = 0;
-  size_t part_rows = 0;    // kv_heads x query_blocks x max_chunks x rows per work-group
+  int32_t part_blocks = 0; // query blocks per subset that may have several chunks
+  size_t part_rows = 0;    // subsets x part_blocks x max_chunks x rows per work-group
   size_t part_bytes = 0;   // part_rows x (head_dim f32 partials + 1 f32 LSE)
   float busiest = 0;       // estimate: key blocks of the busiest CU, its fixed costs among them
   bool idle = false;       // a work-group per query block, fewer of them than CUs

@@ -653,6 +653,7 @@ static int prefill_run(const void* q, int32_t q_dtype, const void* k, const void
       p.pair_parts = plan.pair_parts;
       p.max_chunks = plan.max_chunks;
       if (plan.uses_partials()) {
+        p.part_blocks = plan.part_blocks;
         p.part = static_cast<float*>(partials);
         p.lse = p.part + plan.part_rows * (size_t)head_dim;
       }

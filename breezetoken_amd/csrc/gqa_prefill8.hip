@@ -703,7 +703,7 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
       // One chunk of a split query block: normalised partial and LSE of row
       // (wave, query column) for prefill_combine_kernel; the wave's 16 rows
       // are contiguous.
-      const int64_t slot = ((int64_t)ysub * nqb + qblk) * p.max_chunks + chunk;
+      const int64_t slot = ((int64_t)ysub * p.part_blocks + qblk - (nqb - p.part_blocks)) * p.max_chunks + chunk;
       unsigned char* prows = reinterpret_cast<unsigned char*>(p.part + (slot * kRows8 + wave * kQ8) * D);
       store_f32([&](int r) -> unsigned char* { return prows + r * (D * 4); });
       if (g4 == 0) p.lse[slot * kRows8 + wave * kQ8 + i16] = l_run > 0.f ? fast_log2(l_run) + m_ref : -INFINITY;
@@ -790,7 +790,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
   const int nchunks = p.pair_parts > 0 ? pair_chunks(qblk, nqb, p.pair_parts, n_blocks)
                                        : (n_blocks(qblk) + p.kb_chunk - 1) / p.kb_chunk;
   if (nchunks <= 1) return;
-  const int64_t slot0 = ((int64_t)ysub * nqb + qblk) * p.max_chunks;
+  const int64_t slot0 = ((int64_t)ysub * p.part_blocks + qblk - (nqb - p.part_blocks)) * p.max_chunks;
   const int t = threadIdx.x;
   const int row = (int)blockIdx.z * kRowsPerGroup + t / kD4;
   const int d = (t % kD4) * 4;
@@ -988,7 +988,10 @@ PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv
     plan.busiest = best < nkb_max ? best_cost : whole;
   }
   if (plan.uses_partials()) {
-    plan.part_rows = (size_t)kv_heads * nqb * plan.max_chunks * kRows8;
+    // The longest-first grid cuts its longest query blocks only: slots for
+    // those (H = 8, Hkv = 2, D = 256, S = 4500 44 MB, 74 for all of them).
+    plan.part_blocks = plan.compact == 2 ? longest_second(plan.kb_chunk, seqlen, q_offset, pos_per_wg, nqb, plan.max_chunks) : nqb;
+    plan.part_rows = (size_t)kv_heads * plan.part_blocks * plan.max_chunks * kRows8;
     plan.part_bytes = plan.part_rows * ((size_t)head_dim * 4 + 4);
   }
   return plan;
@@ -1009,7 +1012,8 @@ hipError_t launch_prefill8(const PrefillParams& p, int head_dim, hipStream_t str
   // Partials and the combine (a heavy-first grid of whole query blocks has none).
   const bool split = (p.kb_chunk > 0 && !(p.split_compact == 2 && p.max_chunks == 1)) || (paired && p.max_chunks > 1);
   if (paired && p.kb_chunk > 0) return hipErrorInvalidValue;
-  if (split && (p.max_chunks < 1 || p.max_chunks > kMaxChunks || !p.part || !p.lse)) return hipErrorInvalidValue;
+  if (split && (p.max_chunks < 1 || p.max_chunks > kMaxChunks || p.part_blocks < 1 || !p.part || !p.lse))
+    return hipErrorInvalidValue;
   const int ys = p.kv_heads * p.head_subs;  // grid y: (kv head, head subset)
   const dim3 grid = paired ? dim3(((nqb + 1) / 2) * p.pair_parts, ys, 1)
                    : p.kb_chunk > 0 && p.split_compact == 2

@@ -67,6 +67,27 @@ def test_order_of_whole_query_blocks(steps, heads, kv, dim, q_f32, order):
     assert (got["pair"], got["chunks"], got["order"]) == (0, 1, order)
 
 
+@pytest.mark.parametrize("steps,heads,kv,dim,q_offset", [(4500, 8, 2, 256, 0), (3001, 32, 8, 128, 0), (4200, 8, 2, 256, 300)])
+def test_cut_plan_has_room_for_the_cut_blocks_only(steps, heads, kv, dim, q_offset):
+    """A longest-first grid that cuts query blocks in two keeps partials of those past the cut."""
+    plan = prefill_plan(steps, heads, kv, dim, False, q_offset=q_offset)
+    group = heads // kv
+    pos = 16 * (8 // (group & -group))
+    nqb, subsets = -(-steps // pos), kv * (group // (group & -group))
+    blocks = [-(-(q_offset + min(steps, (b + 1) * pos)) // 64) for b in range(nqb)]
+    if plan["order"] == 2 and plan["chunks"] == 2:
+        cut = sum(n > plan["chunk"] for n in blocks)
+        assert 0 < cut < nqb
+        rows = subsets * cut * 2 * 128
+    else:
+        assert plan["chunks"] == 1
+        rows = 0
+    room = _lib.lib().bt_prefill_partials_bytes(steps, q_offset, heads, kv, dim)
+    assert room == rows * (dim * 4 + 4)
+    if rows:  # one byte less, and the plan is one without partials
+        assert prefill_plan(steps, heads, kv, dim, False, room=room - 1, q_offset=q_offset)["chunks"] == 1
+
+
 def test_plan_refuses_what_the_call_refuses():
     lib, out = _lib.lib(), (ctypes.c_int32 * 5)()
     assert lib.bt_prefill_plan(8, 0, 8, 2, 64, _lib.BT_DTYPE_F32, 0, ctypes.addressof(out)) == _lib.BT_ENOTSUP
