@@ -60,6 +60,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _c_i32,
         [_vp, _c_i32, _c_i32, _c_i32, _vp, _c_i32, _vp, _vp, _vp],
     ),
+    "bt_ragged_plan_cost": (
+        _c_i32,
+        [_vp, _c_i32, _c_i32, _c_i32, _c_i32, _vp, _c_i32, _vp, _vp, _vp],
+    ),
     "bt_ragged_plan_device": (
         ctypes.c_int,
         [_vp, _c_i32, _c_i32, _vp, _c_i32, _vp, _vp, _vp, _vp],
@@ -67,6 +71,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "bt_ragged_plan_rounds_device": (
         ctypes.c_int,
         [_vp, _c_i32, _c_i32, _c_i32, _vp, _c_i32, _vp, _vp, _vp, _vp],
+    ),
+    "bt_ragged_plan_cost_device": (
+        ctypes.c_int,
+        [_vp, _c_i32, _c_i32, _c_i32, _c_i32, _vp, _c_i32, _vp, _vp, _vp, _vp],
     ),
     "bt_gqa_decode_ragged": (
         ctypes.c_int,

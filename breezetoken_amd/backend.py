@@ -375,12 +375,18 @@ class HipBackend:
 
     # ----------------------------------------------------------- ragged decode
     MAX_HOST_PLANS = 64
+    # Fixed cost of a split of a ragged batch, in tokens, by head dimension: with
+    # these the choice between one round of work-groups and several (ragged_groups)
+    # is within 1% of the faster one on average over 553 batches of 4 to 400
+    # sequences of 32 to 32,768 tokens; without, 144 / 200 sequences of 32 to 300
+    # tokens (H = 16, Hkv = 2, D = 256) took 25.4 / 30.6 us instead of 19.6 / 24.4.
+    SPLIT_TOKENS = {64: 120, 128: 150, 256: 300}
 
     def ragged_groups(self, batch: int, kv_heads: int) -> tuple[int, int]:
         """Work-groups per kv head a ragged plan aims for when the caller names
-        none: those of one round (a work-group per CU), used where they are even,
-        and several rounds with room to split the long sequences, used where they
-        are not (bt_ragged_plan_rounds).
+        none: those of one round (a work-group per CU), used where they are even or
+        further splits would cost more than they shorten, and several rounds with
+        room to split the long sequences, used otherwise (bt_ragged_plan_cost).
 
         A batch that (nearly) fills one round keeps one split per sequence, and
         the call lasts as long as one CU takes for its longest sequence: 37 GB/s
@@ -402,18 +408,19 @@ class HipBackend:
         room = max(one, 64, min(batch // 2, 256))
         return one, -(-(batch + room) // one) * one
 
-    def ragged_plan(self, lens: list[int], kv_heads: int, target_groups: int | None = None):
+    def ragged_plan(self, lens: list[int], kv_heads: int, target_groups: int | None = None, split_tokens: int = 0):
         """Split plan for a ragged batch from host lengths, as device tables:
         sequence b gets ceil(len_b / T) splits for the smallest token cap T
         whose total fits ``target_groups`` work-groups per kv head (default:
-        ``ragged_groups``).  Plans are cached per (lens, target), at
+        ``ragged_groups``, with ``split_tokens`` for each further split, as
+        bt_ragged_plan_cost has it).  Plans are cached per (lens, target), at
         most MAX_HOST_PLANS of them (least recently used first out); a plan
         used while a graph is being captured is kept until close()."""
         if target_groups is None:
             one, target = self.ragged_groups(len(lens), kv_heads)
         else:
             one = target = int(target_groups)
-        key = (tuple(int(x) for x in lens), one, target)
+        key = (tuple(int(x) for x in lens), one, target, int(split_tokens) if target != one else 0)
         plan = self._pinned_plans.get(key)
         if plan is None:
             plan = self._plans.get(key)
@@ -430,7 +437,7 @@ class HipBackend:
         return plan
 
     def _host_plan(self, key):
-        lens, one, target = key
+        lens, one, target, split_tokens = key
         batch = len(lens)
         cap = sum(max(1, -(-int(x) // 32)) for x in lens)
         lens_c = (ctypes.c_int32 * batch)(*lens)
@@ -438,12 +445,12 @@ class HipBackend:
         base = (ctypes.c_int32 * batch)()
         count = (ctypes.c_int32 * batch)()
         total = ctypes.c_int32()
-        n = self._lib.bt_ragged_plan_rounds(
-            ctypes.addressof(lens_c), batch, one, target, ctypes.addressof(work), cap,
+        n = self._lib.bt_ragged_plan_cost(
+            ctypes.addressof(lens_c), batch, one, target, split_tokens, ctypes.addressof(work), cap,
             ctypes.addressof(base), ctypes.addressof(count), ctypes.addressof(total),
         )
         if n < 0:
-            check("bt_ragged_plan_rounds", n)
+            check("bt_ragged_plan_cost", n)
         dev = self._dev
         work_t = torch.tensor(list(work)[: 4 * n], dtype=torch.int32).to(dev)
         base_t = torch.tensor(list(base), dtype=torch.int32).to(dev)
@@ -451,14 +458,15 @@ class HipBackend:
         return (work_t, n, base_t, count_t, int(total.value))
 
     def ragged_plan_device(self, seq_len: torch.Tensor, target_groups: int | None = None,
-                           round_groups: int | None = None):
+                           round_groups: int | None = None, split_tokens: int = 0):
         """The same plan built on the device from the device lengths ``seq_len``
         (B,) int32, on the current stream with no host synchronisation
         (capturable).  Tables are allocated once per (B, target) and kept until
         close(); returns (work, num_work, split_base, split_count, total_splits)
         with num_work = total_splits = the table capacity max(B, target).
         ``round_groups`` (at most the target, its default): the plan is for that
-        many work-groups where these are even (bt_ragged_plan_rounds)."""
+        many work-groups where these are even or more splits, of ``split_tokens``
+        tokens' cost each, do not pay (bt_ragged_plan_cost)."""
         batch = int(seq_len.numel())
         if target_groups is None:
             raise ValueError("target_groups is required (CUs / kv heads for one round)")
@@ -476,11 +484,11 @@ class HipBackend:
         work, base, count, total = bufs
         if seq_len.dtype != torch.int32 or seq_len.device != self._dev or not seq_len.is_contiguous():
             raise RuntimeError("seq_len must be a contiguous int32 device tensor")
-        rc = self._lib.bt_ragged_plan_rounds_device(
-            seq_len.data_ptr(), batch, one, target_groups, work.data_ptr(), cap, base.data_ptr(),
+        rc = self._lib.bt_ragged_plan_cost_device(
+            seq_len.data_ptr(), batch, one, target_groups, int(split_tokens), work.data_ptr(), cap, base.data_ptr(),
             count.data_ptr(), total.data_ptr(), _stream(self._dev),
         )
-        check("bt_ragged_plan_rounds_device", rc)
+        check("bt_ragged_plan_cost_device", rc)
         return work, cap, base, count, cap
 
     def attention_ragged(
@@ -503,9 +511,9 @@ class HipBackend:
             one = None
             if target_groups is None:
                 one, target_groups = self.ragged_groups(batch, groups)
-            work, n, base, count, total = self.ragged_plan_device(seq_len, target_groups, one)
+            work, n, base, count, total = self.ragged_plan_device(seq_len, target_groups, one, self.SPLIT_TOKENS[dim])
         else:
-            work, n, base, count, total = self.ragged_plan(lens, groups, target_groups)
+            work, n, base, count, total = self.ragged_plan(lens, groups, target_groups, self.SPLIT_TOKENS[dim])
         ws = self._workspace(heads, dim, total)
         out = torch.empty((batch, heads, dim), dtype=torch.float32, device=self._dev)
         rc = self._lib.bt_gqa_decode_ragged(

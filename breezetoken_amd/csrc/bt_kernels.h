@@ -289,7 +289,16 @@ inline __host__ __device__ bool ragged_round_is_even(int64_t n, int64_t longest,
   return 2 * ((n + round - 1) / round) * longest * round <= 3 * tokens;
 }
 
-// Device-side ragged plan (ragged_plan.hip): the plan bt_ragged_plan_rounds
+// Whether more splits (n2 under a cap of `cap2` tokens, for n and `longest` of
+// one round) pay: what the longest loses, over the CUs of a round, against the
+// fixed cost of the further splits, split_tokens tokens each (prologue, merge,
+// partials through memory).  0: always.  A split has at most cap2 tokens, or 32.
+inline __host__ __device__ bool ragged_splits_pay(int64_t n, int64_t longest, int64_t n2, int64_t cap2,
+                                                  int64_t round, int64_t split_tokens) {
+  return split_tokens == 0 || split_tokens * (n2 - n) <= (longest - (cap2 > 32 ? cap2 : 32)) * round;
+}
+
+// Device-side ragged plan (ragged_plan.hip): the plan bt_ragged_plan_cost
 // makes on the host, from device lengths, padded to work_capacity entries with
 // {-1, ..}.
 constexpr int kRaggedPlanMaxBatch = 4096;
@@ -297,7 +306,8 @@ struct RaggedPlanParams {
   const int32_t* seq_len;  // (batch,) device lengths
   int32_t batch;
   int32_t round_groups;    // work-groups of one round
-  int32_t target_groups;   // work-groups where one round is uneven
+  int32_t target_groups;   // work-groups where one round is uneven and more splits pay
+  int32_t split_tokens;    // fixed cost of a split in tokens (ragged_splits_pay)
   int32_t* work;           // (work_capacity, 4) entries {b, s, ns_b, base_b}
   int32_t work_capacity;   // >= max(batch, target_groups, round_groups)
   int32_t* split_base;     // (batch,)

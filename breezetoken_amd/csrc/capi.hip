@@ -426,8 +426,15 @@ int32_t bt_ragged_plan(const int32_t* lens, int32_t batch, int32_t target_groups
 int32_t bt_ragged_plan_rounds(const int32_t* lens, int32_t batch, int32_t round_groups, int32_t target_groups,
                               int32_t* work, int32_t work_capacity, int32_t* split_base, int32_t* split_count,
                               int32_t* total_splits) {
+  return bt_ragged_plan_cost(lens, batch, round_groups, target_groups, 0, work, work_capacity, split_base,
+                             split_count, total_splits);
+}
+
+int32_t bt_ragged_plan_cost(const int32_t* lens, int32_t batch, int32_t round_groups, int32_t target_groups,
+                            int32_t split_tokens, int32_t* work, int32_t work_capacity, int32_t* split_base,
+                            int32_t* split_count, int32_t* total_splits) {
   if (!lens || !work || !split_base || !split_count || !total_splits) return BT_EINVAL;
-  if (batch < 1 || round_groups < 1 || target_groups < 1) return BT_EINVAL;
+  if (batch < 1 || round_groups < 1 || target_groups < 1 || split_tokens < 0) return BT_EINVAL;
   int32_t max_len = 1;
   int64_t tokens = 0;
   for (int32_t b = 0; b < batch; ++b) {
@@ -468,7 +475,11 @@ int32_t bt_ragged_plan_rounds(const int32_t* lens, int32_t batch, int32_t round_
       const int64_t ns = splits_of(lens[b], cap);
       longest = std::max(longest, (lens[b] + ns - 1) / ns);
     }
-    if (!bt::ragged_round_is_even(count_at(cap), longest, tokens, round_groups)) cap = cap_for(target_groups);
+    const int64_t n = count_at(cap);
+    if (!bt::ragged_round_is_even(n, longest, tokens, round_groups)) {
+      const int32_t more = cap_for(target_groups);
+      if (bt::ragged_splits_pay(n, longest, count_at(more), more, round_groups, split_tokens)) cap = more;
+    }
   }
   int32_t total = 0;
   for (int32_t b = 0; b < batch; ++b) {
@@ -509,14 +520,22 @@ int bt_ragged_plan_device(const int32_t* seq_len, int32_t batch, int32_t target_
 int bt_ragged_plan_rounds_device(const int32_t* seq_len, int32_t batch, int32_t round_groups, int32_t target_groups,
                                  int32_t* work, int32_t work_capacity, int32_t* split_base, int32_t* split_count,
                                  int32_t* total_splits, void* stream) {
+  return bt_ragged_plan_cost_device(seq_len, batch, round_groups, target_groups, 0, work, work_capacity, split_base,
+                                    split_count, total_splits, stream);
+}
+
+int bt_ragged_plan_cost_device(const int32_t* seq_len, int32_t batch, int32_t round_groups, int32_t target_groups,
+                               int32_t split_tokens, int32_t* work, int32_t work_capacity, int32_t* split_base,
+                               int32_t* split_count, int32_t* total_splits, void* stream) {
   if (!seq_len || !work || !split_base || !split_count) return BT_EINVAL;
-  if (batch < 1 || round_groups < 1 || target_groups < 1 || !aligned16(work)) return BT_EINVAL;
+  if (batch < 1 || round_groups < 1 || target_groups < 1 || split_tokens < 0 || !aligned16(work)) return BT_EINVAL;
   if (batch > bt::kRaggedPlanMaxBatch) return BT_ENOTSUP;
   if (work_capacity < std::max(batch, std::max(round_groups, target_groups))) return BT_ENOSPC;
   bt::RaggedPlanParams p{};
   p.seq_len = seq_len;
   p.batch = batch;
   p.round_groups = round_groups;
+  p.split_tokens = split_tokens;
   p.target_groups = target_groups;
   p.work = work;
   p.work_capacity = work_capacity;

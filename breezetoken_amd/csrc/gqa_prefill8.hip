@@ -989,7 +989,7 @@ PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv
   }
   if (plan.uses_partials()) {
     // The longest-first grid cuts its longest query blocks only: slots for
-    // those (H = 8, Hkv = 2, D = 256, S = 4500 44 MB, 74 for all of them).
+    // those (H = 8, Hkv = 2, D = 256, S = 4500 29 MB, 74 for all of them).
     plan.part_blocks = plan.compact == 2 ? longest_second(plan.kb_chunk, seqlen, q_offset, pos_per_wg, nqb, plan.max_chunks) : nqb;
     plan.part_rows = (size_t)kv_heads * plan.part_blocks * plan.max_chunks * kRows8;
     plan.part_bytes = plan.part_rows * ((size_t)head_dim * 4 + 4);

@@ -1,10 +1,11 @@
 // Ragged-batch split plan computed on the device from device lengths, so a
 // multi-sequence decode step needs no host synchronisation and can be captured
-// in a hipGraph.  It makes exactly the plan bt_ragged_plan_rounds (and with
+// in a hipGraph.  It makes exactly the plan bt_ragged_plan_cost (and with
 // round_groups = target_groups, bt_ragged_plan) makes on the host:
 //  * ns_b = ceil(len_b / T), at least 1, at most ceil(len_b / 32) and
 //    kMaxSplitsPerSeq, for the smallest token cap T whose total fits
-//    round_groups, or target_groups where the former leaves the batch uneven;
+//    round_groups, or target_groups where the former leaves the batch uneven and
+//    the further splits pay;
 //  * split_base[b] = sum of ns over sequences before b, split_count[b] = ns_b;
 //  * work entries {b, s, ns_b, base_b}, sequences ordered by tokens per split,
 //    largest first (ties by index, as a stable sort);
@@ -172,11 +173,19 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_plan_kernel(RaggedPlanPar
     tokens += sh.tokens[w];
   }
 
-  int cap = plan_cap(sh, B, p.round_groups, max_len);
+  // Splits under `cap`, their first entries and their total.
+  auto assign = [&](int cap) {
+    const PlanCap T(cap);
+    for (int b = t; b < B; b += kPlanThreads) sh.seq[b].y = T.splits(sh.seq[b].x);
+    __syncthreads();
+    return block_scan(B, sh.base, sh.wave_sum, [&](int b) { return sh.seq[b].y; });
+  };
+  const int cap = plan_cap(sh, B, p.round_groups, max_len);
+  bool one_round = true;
+  int n = 0, longest = 0;
   if (p.target_groups != p.round_groups) {
     // Is one round even enough?  (See ragged_round_is_even.)
     const PlanCap T(cap);
-    int n = 0, longest = 0;
     for (int b = t; b < B; b += kPlanThreads) {
       const int len = sh.seq[b].x, ns = T.splits(len);
       n += ns;
@@ -197,13 +206,18 @@ __global__ __launch_bounds__(kPlanThreads) void ragged_plan_kernel(RaggedPlanPar
       longest = max(longest, sh.longest[w]);
     }
     __syncthreads();
-    if (!ragged_round_is_even(n, longest, tokens, p.round_groups)) cap = plan_cap(sh, B, p.target_groups, max_len);
+    one_round = ragged_round_is_even(n, longest, tokens, p.round_groups);
   }
-
-  const PlanCap T(cap);
-  for (int b = t; b < B; b += kPlanThreads) sh.seq[b].y = T.splits(sh.seq[b].x);
-  __syncthreads();
-  const int total = block_scan(B, sh.base, sh.wave_sum, [&](int b) { return sh.seq[b].y; });
+  int total;
+  if (one_round) {
+    total = assign(cap);
+  } else {
+    // More splits, unless they cost more than they shorten: their number is
+    // known once they are laid out, so that is done first.
+    const int more = plan_cap(sh, B, p.target_groups, max_len);
+    total = assign(more);
+    if (!ragged_splits_pay(n, longest, total, more, p.round_groups, p.split_tokens)) total = assign(cap);
+  }
   // The order of the entries.  Few sequences: each one's rank is counted, the
   // comparisons shared by all threads (B2 threads hold a sequence each, `shares`
   // of them per sequence; lanes of a wave hold one share, so c is uniform).
