@@ -33,6 +33,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "bt_decode_workspace_bytes": (_c_i64, [_c_i32, _c_i32, _c_i32]),
     "bt_decode_pick_splits": (_c_i32, [_c_i32, _c_i32, _c_i32]),
     "bt_decode_pick_splits_batch": (_c_i32, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32]),
+    "bt_decode_pick_splits_uniform": (_c_i32, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32]),
     "bt_gqa_decode_split": (
         ctypes.c_int,
         [_vp, _c_i32, _c_i64, _vp, _vp, _c_i64, _c_i64, _vp, _vp, _vp, _c_i32, _c_i32, _c_i32,

@@ -359,7 +359,8 @@ class HipBackend:
         batch, heads, dim = q.shape
         slots, groups, stride_tok, stride_head = self._kv_layout(k, v, heads, dim)
         q = q.contiguous()
-        ns = int(self._lib.bt_decode_pick_splits_batch(batch, heads, groups, min(int(max_len), 0x7FFFFFFF), self.num_cus))
+        ns = int(self._lib.bt_decode_pick_splits_uniform(batch, heads, groups, dim, min(int(max_len), 0x7FFFFFFF),
+                                                         self.num_cus))
         ws = self._workspace(heads, dim, batch * ns)
         out = torch.empty((batch, heads, dim), dtype=torch.float32, device=self._dev)
         rc = self._lib.bt_gqa_decode(

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <vector>
 
@@ -249,6 +250,51 @@ int32_t bt_decode_pick_splits_batch(int32_t batch, int32_t heads, int32_t kv_hea
     if (cost < best_cost) {
       best = ns;
       best_cost = cost;
+    }
+  }
+  return (int32_t)best;
+}
+
+int32_t bt_decode_pick_splits_uniform(int32_t batch, int32_t heads, int32_t kv_heads, int32_t head_dim,
+                                      int32_t max_len, int32_t num_cus) {
+  if (batch < 1) batch = 1;
+  if (kv_heads < 1) kv_heads = 1;
+  if (heads < kv_heads) heads = kv_heads;
+  if (num_cus < 1) num_cus = 256;
+  if (max_len < 1) max_len = 1;
+  const int64_t pairs = (int64_t)batch * kv_heads, cus = num_cus;
+  const int64_t most = std::min<int64_t>(((int64_t)max_len + 31) / 32, bt::kMaxSplitsPerSeq);
+  // Microseconds of a call with ns splits, lengths between 60% of max_len and all
+  // of it.  Two things bound it together: the tokens the fullest CU streams, at
+  // the rate of one that streams alone, and what all of them move, at 7 TB/s, with
+  // each work-group's fixed time on its CU (one fits a CU at D = 256, two at 128,
+  // three at 64).  More than one split costs the combine's launch and its work.
+  // Fitted to 767 calls at eight shapes, 1 to 128 sequences of 30 to 20,000 tokens.
+  struct Rates {
+    double token, rounds, group;  // a token alone, a round's share of one where there are several, fixed
+  };
+  const Rates r = head_dim > 128  ? Rates{0.0158, 0.7, 1.9}
+                  : head_dim > 64 ? Rates{0.009, 0.84, 0.27}
+                                  : Rates{0.0056, 0.87, 0.06};
+  auto time = [&](int64_t ns) {
+    const double share = std::max(32.0, (double)max_len / (double)ns), n = (double)(pairs * ns);
+    const double rounds = pairs * ns > cus ? r.rounds * (double)((pairs * ns + cus - 1) / cus) : 1.0;
+    const double fullest = rounds * share * r.token + 0.5;
+    const double all = n * (0.8 * share * 4 * head_dim / 7.0e6 + r.group / (double)cus);
+    const double combine = ns > 1 ? 1.8 + 2.5e-5 * (double)batch * heads * head_dim : 0.0;
+    return 3.0 + 0.06 * (heads / kv_heads) + combine + std::sqrt(fullest * fullest + all * all);
+  };
+  // One split, and the counts that fill one to five rounds; more than one round
+  // where it is faster by over 1.5%.
+  const int64_t one = std::max<int64_t>(1, std::min(most, cus / pairs));
+  int64_t best = 1;
+  double best_time = time(1);
+  for (int64_t rounds = 1; rounds <= 5; ++rounds) {
+    const int64_t ns = std::max<int64_t>(1, std::min(most, rounds * cus / pairs));
+    const double t = time(ns) * (ns > one ? 1.015 : 1.0);
+    if (t < best_time) {
+      best = ns;
+      best_time = t;
     }
   }
   return (int32_t)best;

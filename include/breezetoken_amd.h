@@ -66,6 +66,15 @@ int32_t bt_decode_pick_splits(int32_t kv_heads, int32_t ctx_len, int32_t num_cus
 int32_t bt_decode_pick_splits_batch(int32_t batch, int32_t heads, int32_t kv_heads,
                                     int32_t max_len, int32_t num_cus);
 
+/* The same by head dimension too, from rates fitted to it, and never a count that
+ * leaves a few work-groups for a round of their own: what HipBackend takes.
+ * bt_decode_pick_splits_batch splits short sequences and full rounds that are
+ * faster whole: 33 sequences of 300 tokens, H = 32, Hkv = 8, D = 128, 14.5 us in
+ * its 2 splits, 8.8 in one; 128 of 2,000, H = 16, Hkv = 2, D = 256, 86.2 / 70.7;
+ * one of 20,000, H = 8, 12.8 in its 127, 12.1 in 128. */
+int32_t bt_decode_pick_splits_uniform(int32_t batch, int32_t heads, int32_t kv_heads,
+                                      int32_t head_dim, int32_t max_len, int32_t num_cus);
+
 /* Tokens per tile.  The split pass deals tiles to splits round-robin: tile t
  * (tokens [t*T, (t+1)*T)) belongs to split t % num_split.  The reference gives
  * each split a contiguous range instead (attention.py:106-112); the combined
