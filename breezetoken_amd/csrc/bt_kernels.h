@@ -205,40 +205,16 @@ struct GemvParams {
 //    columns and shares of one pass (256 rows), at most 1024 work-groups.  Where
 //    that makes 257..512 of them, a second round that is not full, shares are 512
 //    rows if then all run at once.
-// Two pitches stay with the column kernel: rows that do not begin on a line, where
-// strips share lines, for N and K under 4096 (2560 x 1000 6.57 us against 6.45);
-// and rows of 4 KB from K = 6144, whose strips land on few memory channels (12,288
-// x 2048 13.2 us against 12.1; 8192 x 2048 would gain, 11.9 -> 9.4).
+// Which of these the strip kernel really takes also depends on where W's rows lie
+// (gemv_strips_suit).
 constexpr int kGemvTargetGroups = 512;
 constexpr int kGemvMinRows = 64;
 struct GemvShape {
   int vec, lanes, splits, tiles;
 };
-inline GemvShape gemv_shape(int K, int N) {
+inline GemvShape gemv_column_shape(int K, int N) {
   GemvShape g{};
   const int tiles8 = (N + 511) / 512;
-  if (tiles8 < 256) {
-    const bool narrow = N >= 3072 * ((K + 511) / 512) && N <= 8192;
-    const bool middle = N > (K <= 1024 ? 8192 : 12287) && N <= 16384;
-    const bool wide = N > (K <= 1024 ? 16384 : 24575) && N <= 65536;
-    if (K >= 256 && K <= 1536 && (narrow || middle || wide)) {
-      g.lanes = narrow ? 4 : middle ? 8 : 16;
-      g.tiles = (N + 8 * g.lanes - 1) / (8 * g.lanes);
-      g.splits = 1;
-      return g;
-    }
-    const bool lines = N % 128 == 0 || N >= 4096 || K >= 4096;
-    const bool channels = N != 2048 || K < 6144;
-    if ((K > 2048 || (K > 1024 && N >= 4096)) && lines && channels && N <= 32768) {
-      g.lanes = 16;
-      g.tiles = (N + 127) / 128;
-      const int one = (K + 255) / 256, two = (K + 511) / 512, cap = 1024 / g.tiles;
-      const int64_t groups = (int64_t)g.tiles * one;
-      const int sk = groups > 256 && groups <= 512 && g.tiles * two <= 256 ? two : one;
-      g.splits = sk < cap ? sk : cap;
-      return g;
-    }
-  }
   g.vec = tiles8 >= 8 ? 8 : 4;
   g.tiles = (N + 64 * g.vec - 1) / (64 * g.vec);
   g.splits = 1;
@@ -248,11 +224,74 @@ inline GemvShape gemv_shape(int K, int N) {
   g.splits = sk < 1 ? 1 : (sk > cap ? cap : sk);
   return g;
 }
+// lanes = 0 outside the sizes above.
+inline GemvShape gemv_strip_shape(int K, int N) {
+  GemvShape g{};
+  if (N > 65536) return g;
+  const bool narrow = N >= 3072 * ((K + 511) / 512) && N <= 8192;
+  const bool middle = N > (K <= 1024 ? 8192 : 12287) && N <= 16384;
+  const bool wide = N > (K <= 1024 ? 16384 : 24575);
+  if (K >= 256 && K <= 1536 && (narrow || middle || wide)) {
+    g.lanes = narrow ? 4 : middle ? 8 : 16;
+    g.tiles = (N + 8 * g.lanes - 1) / (8 * g.lanes);
+    g.splits = 1;
+  } else if ((K > 2048 || (K > 1024 && N >= 4096)) && N <= 32768) {
+    g.lanes = 16;
+    g.tiles = (N + 127) / 128;
+    const int one = (K + 255) / 256, two = (K + 511) / 512, cap = 1024 / g.tiles;
+    const int64_t groups = (int64_t)g.tiles * one;
+    const int sk = groups > 256 && groups <= 512 && g.tiles * two <= 256 ? two : one;
+    g.splits = sk < cap ? sk : cap;
+  }
+  return g;
+}
+// Whether the strip kernel is the faster one for a W whose rows begin at `base` and
+// lie `pitch` bytes apart; us, column kernel / strips.
+//  * Rows that do not begin on a line (half a line for strips of 32 columns): each
+//    strip's lines are fetched by its neighbours too, so the column kernel keeps
+//    them: 1536 x 16,392 13.1 / 16.1, 3072 x 16,392 21.7 / 25.8, 2560 x 1024 in a
+//    pitch of 1032 columns 6.35 / 6.53, 4096 x 4104 12.1 / 12.6, 16,384 x 2056 19.3 /
+//    21.6.  Not where the column kernel has few rows per work-group or few
+//    work-groups: K up to 512 (512 x 16,392 0.79 of its time, 50,008 0.96, 65,528
+//    1.08) and 768 in narrow strips (0.82 to 0.96; 1024 1.00 to 1.03); K up to 1280
+//    where its tiles fill a round badly, 18,433 to 28,672 columns (1024 x 19,432 /
+//    24,584 0.86 / 0.87; 768 x 20,008 1.03); tall ones from K = 5120 up to 1536
+//    columns (0.63 to 0.90) and of 2049 to 4095 columns and K = 4096 to 8191 (0.79 to
+//    0.96).
+//  * Rows of whole 4 KB with 1025 to 2048 columns land a strip on few memory
+//    channels: K = 6144 / 10,240 / 12,288 x 2048 8.4 / 8.7, 10.9 / 12.4, 12.2 / 13.2
+//    (pitch 4 KB), 4096 and 6144 in 8 KB 7.7 / 8.0, 8.6 / 9.3; but a power of two of
+//    rows puts the column kernel's 64 shares on few of them as well: 8192 x 2048 11.8
+//    / 9.5, 16,384 x 2048 in 8 KB 22.9 / 17.9.  In a pitch of 2112 columns the strips
+//    take 0.97 to 1.02 of the column kernel's time.
+inline bool gemv_strips_suit(const GemvShape& strip, int K, int N, int64_t pitch, uint64_t base) {
+  const int line = strip.lanes == 4 ? 64 : 128;
+  if (((uint64_t)pitch | base) % line) {
+    if (strip.splits == 1) {
+      if (K <= 512) return N <= 57344;
+      return strip.lanes == 4 ? K <= 768 : K <= 1280 && N > 18432 && N <= 28672;
+    }
+    return N <= 1536 ? K >= 5120 : N > 2048 && N < 4096 && K >= 4096 && K < 8192;
+  }
+  if (N > 1024 && N <= 2048 && pitch % 4096 == 0) {
+    const int long_pitch = pitch % 8192 == 0;
+    const bool two_power = (K & (K - 1)) == 0 && K >= (long_pitch ? 16384 : 8192);
+    return K < (long_pitch ? 4096 : 6144) || two_power;
+  }
+  return true;
+}
+inline GemvShape gemv_shape(int K, int N, int64_t pitch, uint64_t base) {
+  const GemvShape strip = gemv_strip_shape(K, N);
+  return strip.lanes && gemv_strips_suit(strip, K, N, pitch, base) ? strip : gemv_column_shape(K, N);
+}
 
-// Workspace of the split-K matvec: the partial rows.
+// Workspace of the split-K matvec, the partial rows, for any pitch: of the kernel
+// with more shares.
 inline size_t gemv_workspace_bytes(int K, int N) {
-  const GemvShape g = gemv_shape(K, N);
-  return g.splits == 1 ? 0 : (size_t)g.splits * N * 4;
+  const GemvShape strip = gemv_strip_shape(K, N);
+  int splits = gemv_column_shape(K, N).splits;
+  if (strip.lanes && strip.splits > splits) splits = strip.splits;
+  return splits == 1 ? 0 : (size_t)splits * N * 4;
 }
 
 // Keys per block of the prefill key loop, and the size of the transposed,

@@ -883,13 +883,23 @@ int64_t bt_gemv_workspace_bytes(int32_t K, int32_t N) {
   return (int64_t)bt::gemv_workspace_bytes(K, N);
 }
 
+int bt_gemv_plan(const void* w, int64_t ldw, int32_t K, int32_t N, int32_t* plan) {
+  if (!plan || K < 1 || N < 1 || ldw < N) return BT_EINVAL;
+  if (N % 8 || ldw % 8 || !aligned16(w)) return BT_EINVAL;
+  const bt::GemvShape g = bt::gemv_shape(K, N, ldw * 2, reinterpret_cast<uintptr_t>(w));
+  plan[0] = g.lanes > 0 ? 1 : 0;
+  plan[1] = g.lanes > 0 ? 8 * g.lanes : 64 * g.vec;
+  plan[2] = g.splits;
+  return BT_OK;
+}
+
 int bt_gemv_bf16(const float* x, const void* w, int64_t ldw, int32_t K, int32_t N, float* y,
                  void* workspace, int64_t workspace_bytes, void* stream) {
   if (!x || !w || !y || K < 1 || N < 1 || ldw < N) return BT_EINVAL;
   if (N % 8 || ldw % 8 || !aligned16(w)) return BT_EINVAL;
   if ((int64_t)K * ldw * 2 > (int64_t)INT32_MAX) return BT_ENOTSUP;
-  const bt::GemvShape shape = bt::gemv_shape(K, N);
-  const int64_t need = (int64_t)bt::gemv_workspace_bytes(K, N);
+  const bt::GemvShape shape = bt::gemv_shape(K, N, ldw * 2, reinterpret_cast<uintptr_t>(w));
+  const int64_t need = (int64_t)shape.splits * N * 4;
   if (shape.splits > 1 && (!workspace || !aligned16(workspace) || workspace_bytes < need)) return BT_ENOSPC;
   bt::GemvParams p{};
   p.x = x;

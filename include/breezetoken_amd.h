@@ -343,6 +343,11 @@ int bt_gdn_decode(const float* q, const float* k, const float* v, const float* g
  * reference's per-shape partial buffer (backends.py:327). */
 int64_t bt_gemv_workspace_bytes(int32_t K, int32_t N);
 
+/* How bt_gemv_bf16 runs a weight at this address and row stride, without reading
+ * it: plan[0] 1 for the strip kernel, 0 for the column kernel; plan[1] its columns
+ * per work-group; plan[2] its shares of K.  No reference counterpart. */
+int bt_gemv_plan(const void* w, int64_t ldw, int32_t K, int32_t N, int32_t* plan);
+
 /* Decode matvec y (N,) f32 = x (K,) f32 . w (K, N) bf16, w row-major with row
  * stride ldw elements.  Replaces Backend.linear (breezetoken/backends.py:36-37;
  * torch form 182-184) as served by the split-K bf16 GEMV of
