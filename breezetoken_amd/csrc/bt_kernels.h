@@ -249,34 +249,41 @@ inline GemvShape gemv_strip_shape(int K, int N) {
 // lie `pitch` bytes apart; us, column kernel / strips.
 //  * Rows that do not begin on a line (half a line for strips of 32 columns): each
 //    strip's lines are fetched by its neighbours too, so the column kernel keeps
-//    them: 1536 x 16,392 13.1 / 16.1, 3072 x 16,392 21.7 / 25.8, 2560 x 1024 in a
-//    pitch of 1032 columns 6.35 / 6.53, 4096 x 4104 12.1 / 12.6, 16,384 x 2056 19.3 /
-//    21.6.  Not where the column kernel has few rows per work-group or few
-//    work-groups: K up to 512 (512 x 16,392 0.79 of its time, 50,008 0.96, 65,528
-//    1.08) and 768 in narrow strips (0.82 to 0.96; 1024 1.00 to 1.03); K up to 1280
-//    where its tiles fill a round badly, 18,433 to 28,672 columns (1024 x 19,432 /
-//    24,584 0.86 / 0.87; 768 x 20,008 1.03); tall ones from K = 5120 up to 1536
-//    columns (0.63 to 0.90) and of 2049 to 4095 columns and K = 4096 to 8191 (0.79 to
-//    0.96).
-//  * Rows of whole 4 KB with 1025 to 2048 columns land a strip on few memory
-//    channels: K = 6144 / 10,240 / 12,288 x 2048 8.4 / 8.7, 10.9 / 12.4, 12.2 / 13.2
-//    (pitch 4 KB), 4096 and 6144 in 8 KB 7.7 / 8.0, 8.6 / 9.3; but a power of two of
-//    rows puts the column kernel's 64 shares on few of them as well: 8192 x 2048 11.8
-//    / 9.5, 16,384 x 2048 in 8 KB 22.9 / 17.9.  In a pitch of 2112 columns the strips
-//    take 0.97 to 1.02 of the column kernel's time.
+//    most of them: 1536 x 16,392 13.1 / 16.1, 3072 x 16,392 21.7 / 25.8, 2560 x 1024
+//    in a pitch of 1032 columns 6.35 / 6.53, 4096 x 4104 12.1 / 12.6, 16,384 x 2056
+//    19.3 / 21.6.  Strips are still the faster ones
+//    - unsplit: K up to 512 (512 x 16,392 0.79 of the column kernel's time, 50,008
+//      0.96, 65,528 1.08), 768 in narrow strips (0.82 to 0.96; 1024 1.00 to 1.03),
+//      1024 between 18,433 and 32,768 columns, which fill its rounds badly (1024 x
+//      19,432 / 24,584 0.86 / 0.87; 32,776 1.02);
+//    - in shares: where the column kernel's tiles do not fill 512 work-groups evenly
+//      and a few run in a second round, up to 8192 columns (8192 x 1672 15.1 / 10.5,
+//      5120 x 3000 13.5 / 11.0, 6144 x 5128 22.5 / 19.3), one of them only with K under
+//      8192 / 4096 (5120 x 2056 12.1 / 9.6, 2304 x 4104 9.9 / 8.9); from K = 4608 up to 1536
+//      columns always (0.63 to 0.90).
+//  * A pitch of whole 4 KB and 1921 to 2048 columns, 16 strips, which past K = 8192
+//    take a second round and land on few memory channels, while eight column tiles
+//    fill one round: 8453 / 10,240 / 12,288 x 2048 10.9 / 12.1, 11.2 / 12.9, 12.5 / 13.8
+//    (9500 and 11,500 0.92 to 0.97 of the column kernel's time).  Up to there strips
+//    (7000 x 2048 10.7 / 9.3, 8192 11.8 / 9.8), but for whole rows of it in shares of
+//    whole 32-row passes: 6144 x 2048 8.73 / 8.95.  A power of two of rows in 8 KB puts
+//    the column kernel's shares on few channels too: 16,384 x 2048 23.7 / 18.6.
 inline bool gemv_strips_suit(const GemvShape& strip, int K, int N, int64_t pitch, uint64_t base) {
   const int line = strip.lanes == 4 ? 64 : 128;
   if (((uint64_t)pitch | base) % line) {
     if (strip.splits == 1) {
       if (K <= 512) return N <= 57344;
-      return strip.lanes == 4 ? K <= 768 : K <= 1280 && N > 18432 && N <= 28672;
+      return strip.lanes == 4 ? K <= 768 : K <= 1024 && N > 18432 && N <= 32768;
     }
-    return N <= 1536 ? K >= 5120 : N > 2048 && N < 4096 && K >= 4096 && K < 8192;
+    if (K >= 4608 && N <= 1536) return true;
+    const int tiles = gemv_column_shape(K, N).tiles;
+    const int second_round = (kGemvTargetGroups + tiles - 1) / tiles * tiles - kGemvTargetGroups;
+    return N <= 8192 && second_round > 0 && (second_round > 1 || K < (N < 4096 ? 8192 : 4096));
   }
-  if (N > 1024 && N <= 2048 && pitch % 4096 == 0) {
-    const int long_pitch = pitch % 8192 == 0;
-    const bool two_power = (K & (K - 1)) == 0 && K >= (long_pitch ? 16384 : 8192);
-    return K < (long_pitch ? 4096 : 6144) || two_power;
+  if (N > 1920 && N <= 2048 && pitch % 4096 == 0) {
+    const bool two_power = (K & (K - 1)) == 0;
+    if (K > 8192) return two_power && pitch % 8192 == 0;
+    return two_power || K < 6144 || K % 2048 || N * 2 % 4096;
   }
   return true;
 }

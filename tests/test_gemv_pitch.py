@@ -28,6 +28,11 @@ def plan(K, N, ldw, base=1 << 20):
     (16384, 2056, 2056, 0, False),    # 19.3 / 21.6
     (5120, 1032, 1032, 0, True),      # 9.2 / 7.2
     (5120, 3000, 3000, 0, True),      # 13.5 / 11.0
+    (8192, 1672, 1672, 0, True),      # 15.1 / 10.5: seven tiles do not fill a round
+    (8192, 2048, 2056, 0, False),     # eight do
+    (2304, 4104, 4104, 0, True),      # 9.9 / 8.9
+    (6144, 5128, 5128, 0, True),      # 22.5 / 19.3
+    (5120, 2056, 2056, 0, True),      # 12.1 / 9.6
     (512, 16392, 16392, 0, True),     # 0.79 of the column kernel's time
     (512, 65528, 65528, 0, False),    # 1.08
     (768, 6152, 6152, 0, True),       # 0.91
@@ -35,14 +40,16 @@ def plan(K, N, ldw, base=1 << 20):
     (1024, 19432, 19432, 0, True),    # 14.4 / 12.3
     (1024, 6176, 6176, 0, True),      # 0.88: half a line, strips of 32 columns
     (1280, 16448, 16448, 0, True),    # 0.84: 128.5 lines
-    (12288, 2040, 2048, 0, False),    # 12.65 / 13.2: rows of 4 KB
-    (12288, 2048, 2048, 0, False),    # 12.2 / 13.2
-    (6144, 2048, 2048, 0, False),     # 8.4 / 8.7
-    (5120, 2048, 2048, 0, True),      # 9.3 / 8.2
-    (8192, 2048, 2048, 0, True),      # 11.8 / 9.5: a power of two of rows
-    (8192, 2048, 4096, 0, False),     # 10.7 / 10.9, 8 KB
-    (4096, 2048, 4096, 0, False),     # 7.7 / 8.0
-    (16384, 2048, 4096, 0, True),     # 22.9 / 17.9
+    (12288, 2040, 2048, 0, False),    # 13.1 / 13.9: rows of 4 KB
+    (12288, 2048, 2048, 0, False),    # 12.5 / 13.8
+    (8453, 1936, 2048, 0, False),     # 11.3 / 12.1
+    (8453, 1600, 2048, 0, True),      # 13.4 / 9.4: not a full round of the column kernel
+    (6144, 2048, 2048, 0, False),     # 8.73 / 8.95
+    (6144, 2040, 2048, 0, True),      # 9.21 / 8.96
+    (7000, 2048, 2048, 0, True),      # 10.7 / 9.3
+    (8192, 2048, 2048, 0, True),      # 12.1 / 9.9
+    (10240, 2048, 4096, 0, False),    # 11.9 / 14.5, 8 KB
+    (16384, 2048, 4096, 0, True),     # 23.7 / 18.6
     (12288, 2048, 2112, 0, True),     # 12.1 / 12.0
     (8192, 4096, 4096, 0, True),      # 17.2 / 14.9
 ])
@@ -69,8 +76,9 @@ def test_plan_refuses_what_the_call_refuses():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("K,N", [(512, 57344), (512, 57352), (1280, 28672), (1281, 18440), (768, 6152), (776, 6152), (4096, 3000), (8191, 2056),
-                                 (5119, 1536), (5120, 1544), (6144, 1032), (6143, 2048), (8192, 2048), (10240, 2040)])
+@pytest.mark.parametrize("K,N", [(512, 57344), (512, 57352), (1024, 32768), (1025, 18440), (768, 6152), (2056, 8184), (776, 6152), (4096, 3000), (8191, 2056), (8192, 2056),
+                                 (4607, 1000), (4608, 1536), (4608, 1544), (6144, 1032), (6143, 2048), (6144, 2048), (8192, 1800),
+                                 (8193, 2048), (10240, 2040)])
 def test_results_at_each_pitch(hip_backend, K, N):
     gen = torch.Generator(device="cuda").manual_seed(K + N)
     x = torch.randn(K, device="cuda", generator=gen)
