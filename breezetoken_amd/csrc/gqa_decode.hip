@@ -404,12 +404,6 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
                                                          (((st * 4 + kg) ^ (col & (kSlots - 1))) * 16));
 #pragma unroll
       for (int st = 0; st < kSteps; ++st) sacc = mfma16(as_bf16x8(kop[st]), as_bf16x8(qop[st]), sacc);
-      // The scores leave the matrix unit through this fence.  An MFMA's result
-      // may be read 8 wait states after it; hipcc 7.2 counts them over the code
-      // in a row, but where the last MFMA was followed by a branch it put 2 on
-      // the path that takes it, and D = 64 read stale scores.  The nop is tied
-      // to the registers, so nothing that reads them moves ahead of it.
-      asm volatile("s_nop 7" : "+v"(sacc));
     } else {
 #pragma unroll
       for (int st = 0; st < kSteps; ++st) sacc = mfma16(as_bf16x8(kr[st]), as_bf16x8(qop[st]), sacc);
