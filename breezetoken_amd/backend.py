@@ -39,6 +39,7 @@ backends.py:698 with graph.py:127-133).
 from __future__ import annotations
 
 import ctypes
+import operator
 from collections import OrderedDict
 
 import torch
@@ -355,11 +356,12 @@ class HipBackend:
         seq_offset: torch.Tensor, scale: float, max_len: int,
     ) -> torch.Tensor:
         """B sequences sharing one cache, uniform split count; q (B, H, D), pos (B,) int32,
-        seq_offset (B,) int64 first slot of each sequence -> (B, H, D) f32."""
+        seq_offset (B,) int64 first slot of each sequence -> (B, H, D) f32.  ``max_len``
+        (an integer) bounds the lengths for the split count only."""
         batch, heads, dim = q.shape
         slots, groups, stride_tok, stride_head = self._kv_layout(k, v, heads, dim)
         q = q.contiguous()
-        ns = int(self._lib.bt_decode_pick_splits_uniform(batch, heads, groups, dim, min(int(max_len), 0x7FFFFFFF),
+        ns = int(self._lib.bt_decode_pick_splits_uniform(batch, heads, groups, dim, min(operator.index(max_len), 0x7FFFFFFF),
                                                          self.num_cus))
         ws = self._workspace(heads, dim, batch * ns)
         out = torch.empty((batch, heads, dim), dtype=torch.float32, device=self._dev)
