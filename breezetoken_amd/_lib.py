@@ -94,6 +94,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         ctypes.c_int,
         [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i64, _vp],
     ),
+    "bt_prefill_longest_first": (ctypes.c_int, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _vp]),
     "bt_gqa_prefill_cached": (
         ctypes.c_int,
         [_vp, _c_i32, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32,

@@ -370,6 +370,10 @@ hipError_t launch_decode_combine(const CombineParams& p, int head_dim, int heads
 // group runs as subsets of prefill8_sub_group(group) heads.
 bool prefill8_serves(int group, int head_dim);
 int prefill8_sub_group(int group);
+// Work-groups of the longest-first grid (split_compact = 2) of at most two chunks of
+// kb_chunk blocks; item >= 0: that work-group's item too, subset -1 for a padding slot.
+int prefill8_longest_first(int seqlen, int q_offset, int group, int subsets, int kb_chunk, int item, int* subset,
+                           int* qblk, int* chunk);
 // Pair kernel (gqa_prefill_pair.hip): two query blocks per work-group, 32
 // query columns per wave; group sizes 1, 2, 4, 8.
 bool prefill_pair_serves(int group, int head_dim);

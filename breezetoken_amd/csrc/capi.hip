@@ -777,6 +777,21 @@ int bt_prefill_plan(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_
   return BT_OK;
 }
 
+int bt_prefill_longest_first(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads, int32_t kb_chunk,
+                             int32_t item, int32_t* out) {
+  if (!out || seqlen < 1 || q_offset < 0 || heads < 1 || kv_heads < 1 || heads % kv_heads) return BT_EINVAL;
+  if ((int64_t)q_offset + seqlen > INT32_MAX - bt::kPrefillKeyBlock) return BT_EINVAL;
+  const int group = heads / kv_heads, sub = bt::prefill8_sub_group(group);
+  const int nkb = (q_offset + seqlen + bt::kPrefillKeyBlock - 1) / bt::kPrefillKeyBlock;
+  if (group > 8 || kb_chunk < (nkb + 1) / 2 || kb_chunk > nkb) return BT_EINVAL;
+  const int subsets = kv_heads * (group / sub);
+  out[0] = out[1] = out[2] = 0;
+  const int items = bt::prefill8_longest_first(seqlen, q_offset, sub, subsets, kb_chunk, -1, out, out + 1, out + 2);
+  if (item < 0) return items;
+  if (item >= items) return BT_EINVAL;
+  return bt::prefill8_longest_first(seqlen, q_offset, sub, subsets, kb_chunk, item, out, out + 1, out + 2);
+}
+
 int bt_gqa_prefill_cached(const void* q, int32_t q_dtype, const void* k, const void* v, int64_t q_stride_tok,
                           int64_t q_stride_head, int64_t kv_stride_tok, int64_t kv_stride_head, int32_t seqlen,
                           int32_t q_offset, int32_t heads, int32_t kv_heads, int32_t head_dim, float scale,

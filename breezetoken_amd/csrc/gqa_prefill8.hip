@@ -140,6 +140,29 @@ __host__ __device__ inline int longest_ahead(int kb, int S, int P0, int pos, int
 __host__ __device__ inline int longest_second(int kb, int S, int P0, int pos, int nqb, int max_chunks) {
   return max_chunks > 1 ? split_blocks_past(1, kb, S, P0, pos, nqb) : 0;
 }
+// Item L of that grid: its subset, query block and chunk, or false for a padding
+// slot.
+__host__ __device__ inline bool longest_first_item(int L, int kb, int S, int P0, int pos, int nqb, int max_chunks,
+                                                   int subsets, int* subset, int* qblk, int* chunk) {
+  const int ahead = longest_ahead(kb, S, P0, pos, nqb, max_chunks);
+  const int second = longest_second(kb, S, P0, pos, nqb, max_chunks);
+  const int end0 = split_pad8(ahead * subsets), end1 = end0 + split_pad8(second * subsets);
+  int items = ahead * subsets, rank = 0;
+  *chunk = 0;
+  if (L >= end1) {
+    L -= end1;
+    items = (nqb - ahead) * subsets;
+    rank = ahead;
+  } else if (L >= end0) {
+    L -= end0;
+    items = second * subsets;
+    *chunk = 1;
+  }
+  if (L >= items) return false;
+  *subset = L % subsets;
+  *qblk = nqb - 1 - rank - L / subsets;
+  return true;
+}
 inline int longest_first_items(int kb, int S, int P0, int pos, int nqb, int max_chunks, int subsets) {
   const int ahead = longest_ahead(kb, S, P0, pos, nqb, max_chunks);
   return split_pad8(ahead * subsets) + split_pad8(longest_second(kb, S, P0, pos, nqb, max_chunks) * subsets) +
@@ -231,22 +254,8 @@ __global__ __launch_bounds__(kWaves8 * 64, 1) void gqa_prefill8_kernel(PrefillPa
     int L = (int)blockIdx.x;
     bool found = false;
     if (p.split_compact == 2) {
-      const int ahead = longest_ahead(p.kb_chunk, S, P0, pos_per_wg, nqb, p.max_chunks);
-      const int second = longest_second(p.kb_chunk, S, P0, pos_per_wg, nqb, p.max_chunks);
-      const int end0 = split_pad8(ahead * ys), end1 = end0 + split_pad8(second * ys);
-      int items = ahead * ys, rank = 0;
-      if (L >= end1) {
-        L -= end1;
-        items = (nqb - ahead) * ys;
-        rank = ahead;
-      } else if (L >= end0) {
-        L -= end0;
-        items = second * ys;
-        split_chunk = 1;
-      }
-      if (L >= items) return;  // a padding slot (whole work-group)
-      ysub = L % ys;
-      split_qb = nqb - 1 - rank - L / ys;
+      if (!longest_first_item(L, p.kb_chunk, S, P0, pos_per_wg, nqb, p.max_chunks, ys, &ysub, &split_qb, &split_chunk))
+        return;  // a padding slot (whole work-group)
       found = true;
     }
     for (int c = 0; p.split_compact == 1 && c < p.max_chunks && !found; ++c) {
@@ -995,6 +1004,17 @@ PrefillSplitPlan prefill8_split_plan(int seqlen, int q_offset, int group, int kv
     plan.part_bytes = plan.part_rows * ((size_t)head_dim * 4 + 4);
   }
   return plan;
+}
+
+int prefill8_longest_first(int seqlen, int q_offset, int group, int subsets, int kb_chunk, int item, int* subset,
+                           int* qblk, int* chunk) {
+  const int pos_per_wg = kQ8 * (kWaves8 / group);
+  const int nqb = (seqlen + pos_per_wg - 1) / pos_per_wg;
+  const int nkb = (q_offset + seqlen + kKB8 - 1) / kKB8;
+  const int chunks = (nkb + kb_chunk - 1) / kb_chunk;
+  if (item >= 0 && !longest_first_item(item, kb_chunk, seqlen, q_offset, pos_per_wg, nqb, chunks, subsets, subset, qblk, chunk))
+    *subset = -1;
+  return longest_first_items(kb_chunk, seqlen, q_offset, pos_per_wg, nqb, chunks, subsets);
 }
 
 bool prefill8_serves(int group, int head_dim) {

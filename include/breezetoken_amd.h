@@ -273,6 +273,13 @@ int64_t bt_prefill_partials_bytes(int32_t seqlen, int32_t q_offset, int32_t head
 int bt_prefill_plan(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads, int32_t head_dim,
                     int32_t q_dtype, int64_t partials_bytes, int32_t* plan);
 
+/* The grid of a plan with order 2 (bt_prefill_plan), for kb_chunk key blocks per
+ * chunk, at least half of all and at most all: returns its work-groups, or
+ * BT_EINVAL; with item >= 0 also what that one runs, out = {subset of query heads,
+ * query block, chunk}, subset -1 for a padding slot.  No reference counterpart. */
+int bt_prefill_longest_first(int32_t seqlen, int32_t q_offset, int32_t heads, int32_t kv_heads,
+                             int32_t kb_chunk, int32_t item, int32_t* out);
+
 /* bt_gqa_prefill for chunked prefill over one cache, with the K / V^T images
  * kept across calls instead of rebuilt from the whole prefix each time (the
  * chunk loop of Qwen36MoE._attn_batch, breezetoken/model/qwen36_moe.py:

@@ -2,75 +2,86 @@
 work-group per CU or more runs the query blocks of all head subsets longest
 first, the longest ones cut in two where that evens the end.
 
-The device code (gqa_prefill8.hip: split_compact = 2) turns a work-group index
-into (query block, subset, chunk); the arithmetic is restated here and must
-cover every item once, longest first within each region.  The GPU tests run the
-shapes that take the grid, whole and cut, and those whose kernel the estimate
-of capi.hip now chooses (the pair kernel for f32 q from about 1,500 tokens)."""
+bt_prefill_longest_first turns a work-group index into (subset, query block, chunk)
+by the function that the kernel calls; its items must cover every chunk once, in
+their order.  The GPU tests run the shapes that take the grid, whole and cut, and the
+pair kernel for f32 q, and ask the library which of these each one takes."""
 
 from __future__ import annotations
+
+import ctypes
 
 import pytest
 import torch
 
+from breezetoken_amd import _lib
+from test_prefill_choice import ALL, prefill_plan
+
 KB = 64
 
 
-def _past(c, kb, S, P0, pos, nqb):
-    R = c * kb * KB - P0
-    if R < 0:
-        return nqb
-    return 0 if S <= R else nqb - R // pos
+def _items(S, P0, heads, kv, kb):
+    lib, out = _lib.lib(), (ctypes.c_int32 * 3)()
+    total = lib.bt_prefill_longest_first(S, P0, heads, kv, kb, -1, ctypes.addressof(out))
+    assert total > 0
+    for item in range(total):
+        assert lib.bt_prefill_longest_first(S, P0, heads, kv, kb, item, ctypes.addressof(out)) == total
+        yield tuple(out)
 
 
-def _items(kb, S, P0, pos, ys):
-    nqb = -(-S // pos)
-    nkb = (P0 + S + KB - 1) // KB
-    chunks = -(-nkb // kb)
-    assert chunks <= 2
-    ahead = _past(1, nkb - kb, S, P0, pos, nqb) if chunks > 1 and nkb > kb else nqb
-    second = _past(1, kb, S, P0, pos, nqb) if chunks > 1 else 0
-    pad = lambda n: (n + 7) // 8 * 8  # noqa: E731
-    end0 = pad(ahead * ys)
-    end1 = end0 + pad(second * ys)
-    total = end1 + pad((nqb - ahead) * ys)
-    for L in range(total):
-        if L >= end1:
-            at, items, rank, chunk = L - end1, (nqb - ahead) * ys, ahead, 0
-        elif L >= end0:
-            at, items, rank, chunk = L - end0, second * ys, 0, 1
-        else:
-            at, items, rank, chunk = L, ahead * ys, 0, 0
-        if at < items:
-            yield nqb - 1 - rank - at // ys, at % ys, chunk
-
-
-@pytest.mark.parametrize("S,P0,pos,ys", [(4500, 0, 32, 2), (3001, 0, 16, 2), (3001, 0, 32, 8), (700, 3000, 16, 3),
-                                         (1, 0, 16, 5), (2049, 63, 128, 1)])
-def test_items_cover_every_chunk_once(S, P0, pos, ys):
+@pytest.mark.parametrize("S,P0,heads,kv", [(4500, 0, 8, 2), (3001, 0, 16, 2), (3001, 0, 32, 8), (700, 3000, 24, 4),
+                                           (1, 0, 40, 5), (2049, 63, 1, 1), (1500, 0, 6, 2), (130, 8000, 3, 1)])
+def test_items_cover_every_chunk_once(S, P0, heads, kv):
+    group = heads // kv
+    sub = group & -group
+    pos, ys = 16 * (8 // sub), kv * (group // sub)
     nqb, nkb = -(-S // pos), (P0 + S + KB - 1) // KB
-    blocks = lambda qb: (P0 + min(S, (qb + 1) * pos) + KB - 1) // KB  # noqa: E731
+    blocks = [(P0 + min(S, (qb + 1) * pos) + KB - 1) // KB for qb in range(nqb)]
     for kb in sorted({nkb, (nkb + 1) // 2, nkb * 3 // 4, max(1, nkb - 1)}):
         if kb < (nkb + 1) // 2 or kb < 1:
             continue
-        got = list(_items(kb, S, P0, pos, ys))
-        want = {(qb, y, c) for qb in range(nqb) for y in range(ys) for c in range(-(-blocks(qb) // kb))}
+        got = [(qb, y, c) for y, qb, c in _items(S, P0, heads, kv, kb) if y >= 0]
+        want = {(qb, y, c) for qb in range(nqb) for y in range(ys) for c in range(-(-blocks[qb] // kb))}
         assert len(got) == len(set(got)) and set(got) == want
-        # no item starts behind one shorter than half of it (the regions' order)
-        length = [min(kb, blocks(qb) - c * kb) for qb, _, c in got]
-        assert all(a >= b for a, b in zip(length, length[1:]) if a >= nkb - kb > b or a >= kb)
+        # Three runs, each from its longest item: first chunks longer than any second
+        # one, second chunks, the other first chunks.
+        length = {i: min(kb, blocks[i[0]] - i[2] * kb) for i in got}
+        second = [i for i in got if i[2] == 1]
+        at = got.index(second[0]) if second else len(got)
+        runs = [got[:at], second, got[at + len(second):]]
+        assert runs[0] + runs[1] + runs[2] == got
+        for run in runs:
+            assert all(length[a] >= length[b] for a, b in zip(run, run[1:]))
+        if second:
+            top = length[second[0]]
+            assert all(length[i] >= min(top + 1, kb) for i in runs[0]) and all(length[i] <= top for i in runs[2])
+
+
+def test_grid_query_refuses_bad_chunks():
+    lib, out = _lib.lib(), (ctypes.c_int32 * 3)()
+    for kb, item in ((31, -1), (65, -1), (64, 10**6)):  # 64 key blocks in all
+        assert lib.bt_prefill_longest_first(4096, 0, 8, 2, kb, item, ctypes.addressof(out)) == _lib.BT_EINVAL
+    assert lib.bt_prefill_longest_first(4096, 0, 9, 2, 64, -1, ctypes.addressof(out)) == _lib.BT_EINVAL
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("heads,kv,dim,steps,q_f32", [
-    (8, 2, 256, 4500, False),    # cut: 282 work-groups, the longest of 71 blocks
-    (8, 2, 256, 4500, True),
-    (32, 8, 128, 1500, False),   # whole, eight subsets
-    (24, 4, 128, 1400, True),    # three subsets of two heads a kv head
-    (16, 2, 256, 1500, True),    # pair kernel
-    (32, 8, 128, 700, True),     # pair kernel, D = 128
+@pytest.mark.parametrize("heads,kv,dim,steps,q_f32,path,unsplit", [
+    (8, 2, 256, 4500, False, "cut", "subset"),    # 282 work-groups, the longest of 71 blocks
+    (8, 2, 256, 4500, True, "cut", "subset"),
+    (16, 2, 256, 3700, True, "longest", "longest"),  # 232 query blocks a subset: the order over both
+    (32, 8, 128, 1500, False, "longest", "longest"),  # eight subsets
+    (24, 4, 128, 1400, True, "longest", "longest"),   # three subsets of two heads a kv head
+    (16, 2, 256, 1500, True, "pair", "pair"),
+    (32, 8, 128, 700, True, "pair", "pair"),
 ])
-def test_rows_match_the_oracle(hip_backend, heads, kv, dim, steps, q_f32):
+def test_rows_match_the_oracle(hip_backend, heads, kv, dim, steps, q_f32, path, unsplit):
+    if hip_backend.num_cus == 256:
+        for room, want in ((ALL, path), (0, unsplit)):
+            plan = prefill_plan(steps, heads, kv, dim, q_f32, room)
+            kind = ("pair" if plan["pair"] else "cut" if plan["chunks"] == 2 and plan["order"] == 2 else
+                    "longest" if plan["chunks"] == 1 and plan["order"] == 2 else
+                    "subset" if plan["chunks"] == 1 and not plan["parts"] else "other")
+            assert kind == want
     from oracle import attention as orc
 
     print(f"[prefill] H={heads} Hkv={kv} D={dim} S={steps} f32={q_f32}", flush=True)
