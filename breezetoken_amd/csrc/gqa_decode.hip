@@ -55,7 +55,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 constexpr float kDecodeLazy = 8.0f;  // log2-domain slack before the reference max moves
-constexpr int kDecodeEagerTiles = 10;  // tiles per wave up to which a one-split call takes no slack
 
 // K/V are streamed once per call: the non-temporal policy (nt) keeps them from
 // displacing reusable lines and measurably raises the stream rate on gfx950.
@@ -330,16 +329,16 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
     if (threadIdx.x < G) p.lse[(int64_t)(head0 + threadIdx.x) * p.total_splits + split_idx] = -INFINITY;
     return;
   }
-  // A call of one split and a few tiles per wave moves the reference max at
-  // once: its waves' largest probability is then 1, which the bf16 hi + lo pair
-  // holds exactly, as it does where every wave has one tile.  Mean error
-  // against 64 bits over 40 inputs, 1% of the keys scaled by 8, f32 q, with the
-  // slack / without / split over more waves: H = 8, Hkv = 2, D = 256, 301 keys
-  // 4.07 / 4.01 / 4.01e-6; H = 32, Hkv = 8, D = 128, 640 keys 4.69 / 4.62 /
-  // 4.62e-6.  The time is the same (8.8 us a call at 301 keys); with many tiles
-  // per wave the rescales would not be free.
-  float lazy = kDecodeLazy;
-  if constexpr (MODE != kModeRagged) lazy = ns == 1 && tiles <= kDecodeEagerTiles * W ? 0.f : kDecodeLazy;
+  // A sequence of one split moves the reference max at once: its waves' largest
+  // probability is then 1, which the bf16 hi + lo pair holds exactly, as it does
+  // where every wave has one tile; with the slack it may lie anywhere in [1, 2^8].
+  // Mean error against 64 bits, 1% of the keys scaled by 8, f32 q, with the slack /
+  // without / split over more waves: H = 8, Hkv = 2, D = 256, 301 keys 4.07 / 4.01 /
+  // 4.01e-6; unit keys, batches of 56 x 4647 (H = 32, Hkv = 8, D = 128) and 128 x 3000
+  // (H = 16, Hkv = 2, D = 256) 3.48 / 3.24 / 3.47 and 3.45 / 3.19 / 3.40e-6.  The
+  // rescales hide behind the stream: 143.9 / 144.0 and 104.6 / 104.4 us, one split of
+  // 20,000 keys 356.7 / 356.1.
+  const float lazy = ns == 1 ? 0.f : kDecodeLazy;
   const int tstride = ns_eff * W;                       // tile distance between a wave's steps
   const int tfirst = s + ns_eff * wave;                 // this wave's first tile
   // ---- Q^T operand (bf16 hi or lo of q*scale*log2e): wave w builds d-step w.
@@ -444,8 +443,9 @@ __global__ __launch_bounds__(W * 64, 1) void gqa_decode_split_kernel(DecodeSplit
     tmax = halves_fmaxf(tmax);
     // Lazy reference max: m_run moves only when a score exceeds it by more
     // than 2^8 (log2 domain), so p <= 2^8 and O / l are rescaled only then --
-    // behind a wave-uniform branch, almost never after the first tile (short
-    // one-split calls take no slack, see `lazy`).  The LSE stays exact: lse = log2(l) + m_run for whatever reference m_run is.
+    // behind a wave-uniform branch, almost never after the first tile (sequences
+    // of one split take no slack, see `lazy`).  The LSE stays exact: lse = log2(l)
+    // + m_run for whatever reference m_run is.
     // While every score so far is masked, m_run is -inf and does not move
     // (-inf > -inf + 8 is false); subtracting 0 then makes exp2 see -inf
     // (not NaN), so p = 0 acts on an O and l that are 0.

@@ -64,9 +64,9 @@ def test_batch_single_split_rows_and_empty_sequences(hip_backend, out_dtype):
 @pytest.mark.parametrize("seq", [1279, 1280, 1281, 1300])
 @pytest.mark.parametrize("heads,kv,dim", [(8, 2, 256), (6, 2, 64)])
 def test_single_split_around_the_last_slackless_length(hip_backend, heads, kv, dim, seq):
-    """Up to 10 tiles per wave the reference max moves at once, past them with slack: the
-    results on both sides of the line are right where the maximum moves often (what the
-    slack costs is far below this bound; see the test of the mean error)."""
+    """Around 10 tiles per wave, where the reference max moves often (it moves at once at
+    every length of a one-split call; what slack would cost is far below this bound, see the
+    test of the mean error)."""
     case = wl.decode_inputs(37, heads, kv, dim, seq, seq)
     q, k, v = case.q.float(), case.k.clone(), case.v
     k[torch.arange(0, seq, 97)] *= 8.0  # the maximum moves often
@@ -79,12 +79,12 @@ def test_single_split_around_the_last_slackless_length(hip_backend, heads, kv, d
     assert err <= 4e-3 and cos >= 0.99999, (err, cos)
 
 
-def test_mean_error_of_short_one_split_calls(hip_backend):
+@pytest.mark.parametrize("seq,splits", [(301, 10), (3000, 47)])
+def test_mean_error_of_one_split_calls(hip_backend, seq, splits):
     """The slack of the reference max leaves a wave's largest probability off 1, which costs
-    1.5% of the mean error (H = 8, Hkv = 2, D = 256, 301 keys, 1% of them scaled by 8): calls
-    of up to 10 tiles a wave go without, and are no further off than the same call in as many
-    splits as it has tiles, where every wave's maximum is its only one."""
-    heads, kv, dim, seq, err = 8, 2, 256, 301, [0.0, 0.0]
+    0.6 to 1.5% of the mean error (H = 8, Hkv = 2, D = 256, 1% of the keys scaled by 8): calls of one
+    split go without, and are no further off than the same call in more splits."""
+    heads, kv, dim, err = 8, 2, 256, [0.0, 0.0]
     for seed in range(40):
         g = torch.Generator(device="cuda").manual_seed(seed)
         q = torch.randn(heads, dim, device="cuda", generator=g)
@@ -93,8 +93,9 @@ def test_mean_error_of_short_one_split_calls(hip_backend):
         kd, vd = (t.double().repeat_interleave(heads // kv, dim=1).transpose(0, 1) for t in (k, v))
         p = torch.softmax((kd * q.double()[:, None]).sum(-1) * dim**-0.5, dim=-1)
         ref = (p[..., None] * vd).sum(1)
-        for i, splits in enumerate((1, 10)):
-            out = hip_backend.combine(*hip_backend.decode_partials(q, k, v, dim**-0.5, splits))
+        for i, ns in enumerate((1, splits)):
+            out = hip_backend.combine(*hip_backend.decode_partials(q, k, v, dim**-0.5, ns))
             err[i] += ((out.double() - ref).norm() / ref.norm()).item() / 40
-    # Both means scatter together (same inputs); half of what the slack would add.
-    assert err[0] <= 1.0075 * err[1], err
+    # Same inputs on both sides, fixed seeds: 1.0014 and 1.0003 without the slack, 1.0159 and
+    # 1.0062 with it.
+    assert err[0] <= 1.004 * err[1], err
