@@ -547,8 +547,10 @@ class HipBackend:
         strides) -> (S, H, D); row i attends keys
         0 .. q_offset + i.  q_offset = 0 is the SDPA call of prefill.py:56-68, a
         positive one the banded-mask chunked prefill of qwen36_moe.py:394-428.
-        ``split_keys=False`` hands the library only the image workspace, which keeps
-        one work-group per query block (for comparisons; results agree to ~1e-6).
+        ``split_keys=False`` hands the library only the image workspace, without room
+        for partials: whole query blocks, or the pair kernel where that is faster
+        (for comparisons; P is rounded to fp16 at other points, results agree to a
+        few 1e-4).
         ``images`` (a ``PrefillImages`` of this cache) keeps the K / V^T images
         across the chunks of one sequence, so each call converts only the
         blocks from its own first key on; results equal the call without it."""

@@ -21,8 +21,9 @@
 //    bf16; the two halves are summed with one DPP mirror.  P is split the same
 //    way for the P.V product;
 //  * S^T = K . Q^T puts the K tile in the A operand.  K is read in whole token
-//    rows and turned into that layout through the wave's LDS tile; calls with few
-//    tiles per wave read it straight into registers in the operand layout instead
+//    rows and turned into that layout through the wave's LDS tile; calls by device
+//    position at D = 256 with groups of up to 4 heads, one split or a cache under
+//    16,384 slots read it straight into registers in the operand layout instead
 //    (64 contiguous bytes per token per instruction).  Loads are 16-byte buffer
 //    loads; those past the valid length return zero (buffer bounds);
 //  * V is staged through an XOR-swizzled LDS tile per wave and read back with
@@ -696,7 +697,8 @@ __global__ __launch_bounds__(64) void gqa_decode_combine_kernel(CombineParams p)
 // position at D = 256 where waves get too few tiles for the better stream to pay
 // for the LDS pass: groups of up to 4 heads, one split, caches under 16,384
 // slots.  us per call, pieces -> rows: H = 16, Hkv = 2, D = 256 at 32k / 131k
-// 17.85 / 49.9 -> 16.9 / 48.2; H = 32, Hkv = 8, D = 128 at 4k / 32k 8.9 / 28.6 ->
+// 17.85 / 49.9 -> 16.9 / 48.2 eager, 16.43 / 46.00 -> 16.39 / 46.74 by position in a
+// graph over six caches; H = 32, Hkv = 8, D = 128 at 4k / 32k 8.9 / 28.6 ->
 // 8.6 / 25.5; ragged 32 x 256 .. 32,768 tokens, D = 256, 83.7 -> 77.8, 24 x 256
 // .. 4,000, D = 128, 39.7 -> 36.0.  H = 8, Hkv = 2, D = 256 by position gains 1%
 // at 32k (15.9 -> 15.7) and loses 2% at 1k and 4k (6.65 -> 6.75, 7.40 -> 7.54).
